@@ -83,8 +83,9 @@ int w4a8_quant_per_token(const void* x, long ldx, void* q, float* scale, int M, 
                          void* stream);
 
 /* (2) One-time weight repack: checkpoint w [N, K/2] + ws [N, K/32] -> wq, sq (w4a8_packed_bytes).
- * Out of place; the caller may copy the result back into the checkpoint storage when the sizes
- * match. Replaces the load-time repack of process_weights_after_loading: scale transpose,
+ * Out of place, or in place (wq == w, sq == ws) when there is nothing to pad and each n-tile fits
+ * one workgroup's LDS: N % 16 == 0, K % 512 == 0, K <= 19968, ws 16-byte aligned; other
+ * overlap of input and output is not supported. Replaces the load-time repack of process_weights_after_loading: scale transpose,
  * make_row_ref, permute_w, psw_pack_w_, psw_fold_ws (sly/mxfp4/radiance_mxfp4.py:1083-1171). */
 int w4a8_repack(const void* w, const void* ws, void* wq, void* sq, int N, int K, void* stream);
 

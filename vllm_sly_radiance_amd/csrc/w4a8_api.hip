@@ -574,6 +574,9 @@ W4A8_API int w4a8_repack(const void* w, const void* ws, void* wq, void* sq, int 
   if (!w || !ws || !wq || !sq) return fail(W4A8_EINVAL, "w4a8_repack: null pointer");
   if (!aligned(w, 16) || !aligned(wq, 16) || !aligned(sq, 4))
     return fail(W4A8_EINVAL, "w4a8_repack: w and wq need 16-byte alignment, sq 4-byte");
+  if ((w == wq || ws == sq) && !repack_in_place((const uint8_t*)ws, N, K))
+    return fail(W4A8_EINVAL, "w4a8_repack: in place needs N %% 16 == 0, K %% 512 == 0, K <= 19968 "
+                "and 16-byte aligned ws (N=%d K=%d)", N, K);
   return hip_status(launch_repack((const uint8_t*)w, (const uint8_t*)ws, (uint8_t*)wq,
                                   (uint32_t*)sq, N, K, (hipStream_t)stream),
                     "w4a8_repack");

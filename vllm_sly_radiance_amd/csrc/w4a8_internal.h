@@ -119,6 +119,8 @@ struct GemmArgs {
 
 hipError_t launch_quant(const uint16_t* x, long ldx, uint8_t* q, float* s, int M, int K,
                         hipStream_t stream);
+// the repack reads each n-tile whole before it writes it: w == wq and ws == sq are then allowed
+bool repack_in_place(const uint8_t* ws, int N, int K);
 hipError_t launch_repack(const uint8_t* w, const uint8_t* ws, uint8_t* wq, uint32_t* sq, int N,
                          int K, hipStream_t stream);
 // tiled: q is written fragment-tiled (K or N a multiple of 128) instead of row-major

@@ -70,9 +70,14 @@ def quant_per_token(x: torch.Tensor):
     return q, s
 
 
-def repack_weights(weight: torch.Tensor, weight_scale: torch.Tensor):
+# Widest K whose n-tiles the repack holds in one workgroup's LDS, and so rewrites in place.
+REPACK_IN_PLACE_MAX_K = 19968
+
+
+def repack_weights(weight: torch.Tensor, weight_scale: torch.Tensor, in_place: bool = False):
     """Checkpoint (weight [N, K/2] uint8, weight_scale [N, K/32] uint8) -> granules (wq, sq) as
-    uint8 [Np, Kp/2] and [Np, Kp/32]."""
+    uint8 [Np, Kp/2] and [Np, Kp/32]. in_place lets the granules overwrite the inputs where nothing
+    is padded (contiguous inputs then come back as they are, rewritten)."""
     N, K = weight.shape[0], weight.shape[1] * 2
     if weight.dtype != torch.uint8 or weight_scale.dtype != torch.uint8 \
             or tuple(weight_scale.shape) != (N, K // 32):
@@ -83,8 +88,12 @@ def repack_weights(weight: torch.Tensor, weight_scale: torch.Tensor):
     ws = weight_scale.contiguous()
     wq_bytes, sq_bytes = _native.packed_bytes(N, K)
     Np, Kp = -(-N // 16) * 16, -(-K // 512) * 512
-    wq = torch.empty((Np, Kp // 2), dtype=torch.uint8, device=w.device)
-    sq = torch.empty((Np, Kp // 32), dtype=torch.uint8, device=w.device)
+    if in_place and (Np, Kp) == (N, K) and K <= REPACK_IN_PLACE_MAX_K \
+            and w.data_ptr() % 16 == 0 and ws.data_ptr() % 16 == 0:
+        wq, sq = w, ws
+    else:
+        wq = torch.empty((Np, Kp // 2), dtype=torch.uint8, device=w.device)
+        sq = torch.empty((Np, Kp // 32), dtype=torch.uint8, device=w.device)
     assert wq.numel() == wq_bytes and sq.numel() == sq_bytes
     _native.repack(w.data_ptr(), ws.data_ptr(), wq.data_ptr(), sq.data_ptr(), N, K, _stream())
     return wq, sq
@@ -399,13 +408,17 @@ def _make_kernel_class():
                     f"{layer.weight.dtype} / weight_scale {tuple(layer.weight_scale.shape)} is not "
                     f"an MXFP4 checkpoint layer this kernel serves")
             ensure_scratch(layer.weight.device)
-            wq, sq = repack_weights(layer.weight.data, layer.weight_scale.data)
+            # where nothing is padded the repack rewrites the checkpoint storage itself: no second
+            # copy of the layer, no copy back, no allocator holes
+            wq, sq = repack_weights(layer.weight.data, layer.weight_scale.data, in_place=True)
             if wq.shape == layer.weight.shape and layer.weight.is_contiguous():
-                layer.weight.data.copy_(wq)              # same storage: no allocator holes
+                if wq.data_ptr() != layer.weight.data_ptr():
+                    layer.weight.data.copy_(wq)
             else:
                 layer.weight = torch.nn.Parameter(wq, requires_grad=False)
             if sq.shape == layer.weight_scale.shape and layer.weight_scale.is_contiguous():
-                layer.weight_scale.data.copy_(sq)
+                if sq.data_ptr() != layer.weight_scale.data_ptr():
+                    layer.weight_scale.data.copy_(sq)
             else:
                 layer.weight_scale = torch.nn.Parameter(sq, requires_grad=False)
             del wq, sq
