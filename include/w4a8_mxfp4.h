@@ -159,8 +159,9 @@ int w4a8_gemm_noalloc(const void* a, const float* a_scale, const void* wq, const
  * tile:   p = {WM, WN (MFMA tiles per wave), BM, BN (workgroup tile)};
  * stream: p = {NT (n-tiles per workgroup at most), KPW (k-tiles per wave at most), waves,
  *         NT * KPW (granules per wave at most)}. A stream variant serves (M, N, K) only when
- *         M <= 16, K % 512 == 0 and the shape's n-tiles per workgroup and k-tiles per wave fit it;
- *         forcing one that does not returns W4A8_EINVAL.
+ *         M <= 16, K % 128 == 0 (at most an eighth of K in padding to 512) and the shape's
+ *         n-tiles per workgroup and k-tiles per wave fit it; forcing one that does not returns
+ *         W4A8_EINVAL.
  * ring:   p = {MF (16-token fragments), NT (n-tiles per workgroup at most), D (k-tile stages in
  *         flight per wave), waves}. A ring variant serves (M, N, K) when M <= 16 * MF, the
  *         shape's n-tiles per workgroup fit NT and every wave owns a k-tile.

@@ -163,7 +163,7 @@ int find_stream(int M, int N, int K, int dev) {
     const StreamCfg c = stream_variant(v);
     const int regs = 4 * c.nt * c.kpw + (M <= 8 ? 4 : 8) * c.kpw;
     const long key =
-        wide && regs <= 160 && c.waves <= K / kKAlign
+        wide && regs <= 160 && c.waves <= padded_k(K) / kKAlign
             ? ((long)c.waves * 4096 + regs) * 64 + c.nt
             : (1L << 40) + ((long)stream_granules(v, N, K, d.cus) * 64 + c.nt) * 64 + c.waves;
     if (best < 0 || key < best_key) best = v, best_key = key;

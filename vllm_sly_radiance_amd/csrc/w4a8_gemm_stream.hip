@@ -60,7 +60,8 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // NT: n-tiles per workgroup at most; KPW: k-tiles per wave at most (a multiple of 4); W: waves.
-// The host requires K % 512 == 0 (whole k-groups), M <= 16 (M <= 8 with H8),
+// The host requires K % 128 == 0 (whole k-tiles; the padding up to whole k-groups is zero weights,
+// and the k-tiles past K re-read the row's last one), M <= 16 (M <= 8 with H8),
 // 4 * ceil(KG / W) <= KPW. H8 (M <= 8): one load per k-tile brings both 16-byte runs of the 8
 // live tokens (lanes 8..15 of each row of 16 load the second run of token r - 8, and a row
 // rotation by 8 lanes hands it to lane r), half the activation loads; the MFMA columns of tokens
@@ -68,13 +69,16 @@ __device__ __forceinline__ void lds_barrier() {
 // The 14 argument dwords are exactly what the kernel arguments preloaded into SGPRs hold, so no
 // wave reads the kernarg segment, not even for the epilogue (whose scalar load used to sit on the
 // critical path after the last MFMA); the n-tile count and the store width follow from N and C.
-template <int NT, int KPW, int W, bool H8>
+template <int NT, int KPW, int W, bool H8, bool TAIL>
 __global__ __launch_bounds__(W * 64) void gemm_stream(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
     const uint32_t* __restrict__ Sq, uint16_t* __restrict__ C, int M, int K, int N, int S) {
   static_assert(KPW % 4 == 0 && NT >= 1 && W >= 1 && W <= 16, "stream variant");
-  // K % 512 == 0; K, N > 0 (unsigned shifts: no sign fix-ups in the scalar prologue)
-  const int KT = (int)((unsigned)K / kKTile), KG = (int)((unsigned)KT / kKGroup);
+  // K % 128 == 0; K, N > 0 (unsigned shifts: no sign fix-ups in the scalar prologue). KT
+  // activation k-tiles; the weights are padded to KTP, whole k-groups, with zeros.
+  const int KT = (int)((unsigned)K / kKTile);
+  const int KG = (int)((unsigned)(TAIL ? KT + kKGroup - 1 : KT) / kKGroup);
+  const int KTP = TAIL ? KG * kKGroup : KT;
   const int NTILES = (int)(((unsigned)N + kNTile - 1) / kNTile);
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -83,8 +87,8 @@ __global__ __launch_bounds__(W * 64) void gemm_stream(
   const int b = blockIdx.x;
   const int ntb0 = b * S, nth = min(S, NTILES - ntb0);
   // the workgroup's first granule stripe and scale rows (one 64-bit product); an n-tile's stripe
-  // is t KT KiB further, below 2^31 for the NT n-tiles of a workgroup (the host checks it)
-  const uint8_t* const wbase = Wq + (size_t)ntb0 * KT * kGranuleBytes;
+  // is t KTP KiB further, below 2^31 for the NT n-tiles of a workgroup (the host checks it)
+  const uint8_t* const wbase = Wq + (size_t)ntb0 * KTP * kGranuleBytes;
   const uint8_t* const sbase = reinterpret_cast<const uint8_t*>(Sq) + (size_t)ntb0 * KG * 256;
   // the epilogue: thread tid adds the partials of output slot tid (below); at M <= 8 a slot is one
   // of the 32 lanes of an n-tile that hold tokens 0..7
@@ -136,7 +140,7 @@ __global__ __launch_bounds__(W * 64) void gemm_stream(
     for (int t = 0; t < NT; ++t) {
       const bool have = t < nth;
       w_src[t] = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)(wbase + (uint32_t)(t * KT * kGranuleBytes)), 0,
+          (void*)(wbase + (uint32_t)(t * KTP * kGranuleBytes)), 0,
           have ? kr1 * kGranuleBytes : 0, kBufferWord3);
       s_src[t] = __builtin_amdgcn_make_buffer_rsrc((void*)(sbase + (uint32_t)(t * KG * 256)), 0,
                                                    have ? (kr1 >> 2) * 256 : 0, kBufferWord3);
@@ -247,21 +251,24 @@ __global__ __launch_bounds__(W * 64) void gemm_stream(
 // goes to out[0] only if it equals a fixed pattern, so the compiler cannot drop a load.
 constexpr int kStreamLoadWeights = 1, kStreamLoadScales = 2, kStreamLoadActivations = 4;
 
-template <int NT, int KPW, int W, int PARTS>
+template <int NT, int KPW, int W, int PARTS, bool TAIL>
 __global__ __launch_bounds__(W * 64) void gemm_stream_loads(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
     const uint32_t* __restrict__ Sq, int* __restrict__ out, int M, int K, int N, int S) {
   static_assert(KPW % 4 == 0 && NT >= 1 && W >= 1 && W <= 16, "stream variant");
-  // K % 512 == 0; K, N > 0 (unsigned shifts: no sign fix-ups in the scalar prologue)
-  const int KT = (int)((unsigned)K / kKTile), KG = (int)((unsigned)KT / kKGroup);
+  // K % 128 == 0; K, N > 0 (unsigned shifts: no sign fix-ups in the scalar prologue). KT
+  // activation k-tiles; the weights are padded to KTP, whole k-groups, with zeros.
+  const int KT = (int)((unsigned)K / kKTile);
+  const int KG = (int)((unsigned)(TAIL ? KT + kKGroup - 1 : KT) / kKGroup);
+  const int KTP = TAIL ? KG * kKGroup : KT;
   const int NTILES = (int)(((unsigned)N + kNTile - 1) / kNTile);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = blockIdx.x;
   const int ntb0 = b * S, nth = min(S, NTILES - ntb0);
   // the workgroup's first granule stripe and scale rows (one 64-bit product); an n-tile's stripe
-  // is t KT KiB further, below 2^31 for the NT n-tiles of a workgroup (the host checks it)
-  const uint8_t* const wbase = Wq + (size_t)ntb0 * KT * kGranuleBytes;
+  // is t KTP KiB further, below 2^31 for the NT n-tiles of a workgroup (the host checks it)
+  const uint8_t* const wbase = Wq + (size_t)ntb0 * KTP * kGranuleBytes;
   const uint8_t* const sbase = reinterpret_cast<const uint8_t*>(Sq) + (size_t)ntb0 * KG * 256;
   const int om = tid & 7;
   const int kr0 = 4 * (int)((unsigned)(KG * wave) / W);
@@ -302,7 +309,7 @@ __global__ __launch_bounds__(W * 64) void gemm_stream_loads(
     for (int t = 0; t < NT; ++t) {
       const bool have = t < nth;
       w_src[t] = __builtin_amdgcn_make_buffer_rsrc(
-          (void*)(wbase + (uint32_t)(t * KT * kGranuleBytes)), 0,
+          (void*)(wbase + (uint32_t)(t * KTP * kGranuleBytes)), 0,
           have ? kr1 * kGranuleBytes : 0, kBufferWord3);
       s_src[t] = __builtin_amdgcn_make_buffer_rsrc((void*)(sbase + (uint32_t)(t * KG * 256)), 0,
                                                    have ? (kr1 >> 2) * 256 : 0, kBufferWord3);
@@ -356,7 +363,7 @@ __global__ __launch_bounds__(W * 64) void gemm_stream_loads(
 // corrected quotient), so the output equals quantizer + GEMM bit for bit.
 // LDS: the codes [k-tile][half][lane group][8 tokens][16 B] (KT KiB), then 8 token scales, three
 // counters, Q x 8 partial maxima (512 B in all), then the partial sums. X is bf16 [M, ldx], 16-byte
-// aligned rows; the host requires M <= 8, 4 <= W <= 12, K % 512 == 0 and 16 ldx < 2^31.
+// aligned rows; the host requires M <= 8, 4 <= W <= 12, K % 128 == 0 and 16 ldx < 2^31.
 // SILU: X is the gate/up output of the layer before, [M, ldx] with gate in columns 0..K-1 and up in
 // K..2K-1, and the row quantized is the SiLU-and-mul producer's bf16 stage,
 // bf16(bf16(silu(gate)) * up), computed with the producer's own steps (w4a8_silu.h); M <= 2.
@@ -390,14 +397,17 @@ __device__ __forceinline__ void fq_signal(int* counter) {
     __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-template <int NT, int KPW, int W, bool SILU>
+template <int NT, int KPW, int W, bool SILU, bool TAIL>
 __global__ __launch_bounds__(kFqWaves * 64) void gemm_stream_fq(
     const uint8_t* __restrict__ X, const uint8_t* __restrict__ Wq, const uint32_t* __restrict__ Sq,
     uint16_t* __restrict__ C, int M, int K, int N, int S, int ldx) {
   constexpr int Q = kFqWaves - W;                // quantizing waves
   static_assert(KPW % 4 == 0 && NT >= 1 && W >= 1 && Q >= 4 && Q <= 12, "fq variant");
-  // K % 512 == 0; K, N > 0 (unsigned shifts: no sign fix-ups in the scalar prologue)
-  const int KT = (int)((unsigned)K / kKTile), KG = (int)((unsigned)KT / kKGroup);
+  // K % 128 == 0; K, N > 0 (unsigned shifts: no sign fix-ups in the scalar prologue). KT
+  // activation k-tiles; the weights are padded to KTP, whole k-groups, with zeros.
+  const int KT = (int)((unsigned)K / kKTile);
+  const int KG = (int)((unsigned)(TAIL ? KT + kKGroup - 1 : KT) / kKGroup);
+  const int KTP = TAIL ? KG * kKGroup : KT;
   const int NTILES = (int)(((unsigned)N + kNTile - 1) / kNTile);
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   uint8_t* const codes = lds;
@@ -411,8 +421,8 @@ __global__ __launch_bounds__(kFqWaves * 64) void gemm_stream_fq(
   const int b = blockIdx.x;
   const int ntb0 = b * S, nth = min(S, NTILES - ntb0);
   // the workgroup's first granule stripe and scale rows (one 64-bit product); an n-tile's stripe
-  // is t KT KiB further, below 2^31 for the NT n-tiles of a workgroup (the host checks it)
-  const uint8_t* const wbase = Wq + (size_t)ntb0 * KT * kGranuleBytes;
+  // is t KTP KiB further, below 2^31 for the NT n-tiles of a workgroup (the host checks it)
+  const uint8_t* const wbase = Wq + (size_t)ntb0 * KTP * kGranuleBytes;
   const uint8_t* const sbase = reinterpret_cast<const uint8_t*>(Sq) + (size_t)ntb0 * KG * 256;
   if (wave >= W) {
     // ---- quantizing wave q: chunk columns [c0, c1) of every row (a chunk: 8 elements, 16 B),
@@ -496,7 +506,7 @@ __global__ __launch_bounds__(kFqWaves * 64) void gemm_stream_fq(
       for (int t = 0; t < NT; ++t) {
         const bool have = t < nth;
         w_src[t] = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)(wbase + (uint32_t)(t * KT * kGranuleBytes)), 0,
+            (void*)(wbase + (uint32_t)(t * KTP * kGranuleBytes)), 0,
             have ? kr1 * kGranuleBytes : 0, kBufferWord3);
         s_src[t] = __builtin_amdgcn_make_buffer_rsrc(
             (void*)(sbase + (uint32_t)(t * KG * 256)), 0, have ? (kr1 >> 2) * 256 : 0,
@@ -612,10 +622,11 @@ size_t stream_lds_bytes(int variant, int M, int K, bool fused) {
 // Granules the busiest wave of a variant streams for this shape (0: the variant cannot serve it).
 int stream_granules(int variant, int N, int K, int cus) {
   const StreamCfg c = kStream[variant];
-  if (K % 512) return 0;
+  // Whole k-tiles, and at most an eighth of K in zero padding (a wave streams it like the rest).
+  if (K % kKTile || 8 * (padded_k(K) - K) > K) return 0;
   const int ntiles = padded_n(N) / kNTile;
   const int ntmax = ceil_div(ntiles, stream_grid(N, cus));
-  const int kpw = 4 * ceil_div(K / kKAlign, c.waves);
+  const int kpw = 4 * ceil_div(padded_k(K) / kKAlign, c.waves);
   if (ntmax > c.nt || kpw > c.kpw) return 0;
   return ntmax * kpw;
 }
@@ -624,7 +635,7 @@ bool stream_fits(int variant, int M, int N, int K, int cus, size_t lds_limit) {
   if (M < 1 || M > 16 || stream_granules(variant, N, K, cus) == 0) return false;
   const StreamCfg c = kStream[variant];
   // every offset the kernel forms stays in 32 bits
-  const bool small = (long)M * K < (1L << 31) && (long)c.nt * (K / kKTile) * kGranuleBytes <
+  const bool small = (long)M * K < (1L << 31) && (long)c.nt * (padded_k(K) / kKTile) * kGranuleBytes <
                      (1L << 31) && (long)padded_n(N) < (1L << 24);
   return small && stream_lds_bytes(variant, M, K, false) <= lds_limit;
 }
@@ -665,36 +676,39 @@ hipError_t launch_stream(const GemmArgs& g, int variant, int cus, bool fused, lo
                                              (int)lds);                                          \
     if (e != hipSuccess) return e;                                                               \
   }
-#define W4A8_STREAM_GO(nt, kpw, w, h8)                                                           \
+#define W4A8_STREAM_GO(nt, kpw, w, h8, tail)                                                     \
   {                                                                                              \
-    W4A8_STREAM_ATTR((gemm_stream<nt, kpw, w, h8>))                                              \
-    hipLaunchKernelGGL((gemm_stream<nt, kpw, w, h8>), grid, block, lds, stream, g.a, g.a_scale,  \
-                       g.wq, g.sq, g.c, g.M, g.K, g.N, share);                            \
+    W4A8_STREAM_ATTR((gemm_stream<nt, kpw, w, h8, tail>))                                        \
+    hipLaunchKernelGGL((gemm_stream<nt, kpw, w, h8, tail>), grid, block, lds, stream, g.a,       \
+                       g.a_scale, g.wq, g.sq, g.c, g.M, g.K, g.N, share);                        \
+    return hipGetLastError();                                                                    \
+  }
+#define W4A8_STREAM_FQ_GO(nt, kpw, w, silu, tail)                                                \
+  {                                                                                              \
+    W4A8_STREAM_ATTR((gemm_stream_fq<nt, kpw, w, silu, tail>))                                   \
+    hipLaunchKernelGGL((gemm_stream_fq<nt, kpw, w, silu, tail>), grid, dim3(kFqWaves * 64), lds, \
+                       stream, g.a, g.wq, g.sq, g.c, g.M, g.K, g.N, share, (int)lda);            \
     return hipGetLastError();                                                                    \
   }
 #define W4A8_STREAM_LAUNCH(nt, kpw, w)                                                           \
   if (idx++ == variant) {                                                                        \
+    const bool tail = g.K % kKAlign != 0;                                                        \
     if constexpr (w >= 4 && w <= kFqWaves - 4 && nt * kpw <= 24) {                               \
-      if (fused && silu) {                                                                       \
-        W4A8_STREAM_ATTR((gemm_stream_fq<nt, kpw, w, true>))                                     \
-        hipLaunchKernelGGL((gemm_stream_fq<nt, kpw, w, true>), grid, dim3(kFqWaves * 64), lds,    \
-                           stream, g.a, g.wq, g.sq, g.c, g.M, g.K, g.N, share, (int)lda);  \
-        return hipGetLastError();                                                                \
-      }                                                                                          \
-      if (fused) {                                                                               \
-        W4A8_STREAM_ATTR((gemm_stream_fq<nt, kpw, w, false>))                                    \
-        hipLaunchKernelGGL((gemm_stream_fq<nt, kpw, w, false>), grid, dim3(kFqWaves * 64), lds,   \
-                           stream, g.a, g.wq, g.sq, g.c, g.M, g.K, g.N, share, (int)lda);  \
-        return hipGetLastError();                                                                \
-      }                                                                                          \
+      if (fused && silu && tail) W4A8_STREAM_FQ_GO(nt, kpw, w, true, true)                       \
+      if (fused && silu) W4A8_STREAM_FQ_GO(nt, kpw, w, true, false)                              \
+      if (fused && tail) W4A8_STREAM_FQ_GO(nt, kpw, w, false, true)                              \
+      if (fused) W4A8_STREAM_FQ_GO(nt, kpw, w, false, false)                                     \
     }                                                                                            \
     if (fused) return hipErrorInvalidValue;                                                      \
-    if (g.M <= 8) W4A8_STREAM_GO(nt, kpw, w, true)                                               \
-    W4A8_STREAM_GO(nt, kpw, w, false)                                                            \
+    if (g.M <= 8 && tail) W4A8_STREAM_GO(nt, kpw, w, true, true)                                 \
+    if (g.M <= 8) W4A8_STREAM_GO(nt, kpw, w, true, false)                                        \
+    if (tail) W4A8_STREAM_GO(nt, kpw, w, false, true)                                            \
+    W4A8_STREAM_GO(nt, kpw, w, false, false)                                                     \
   }
   W4A8_STREAM_TABLE(W4A8_STREAM_LAUNCH)
 #undef W4A8_STREAM_LAUNCH
 #undef W4A8_STREAM_GO
+#undef W4A8_STREAM_FQ_GO
 #undef W4A8_STREAM_ATTR
   return hipErrorInvalidValue;
 }
@@ -704,18 +718,20 @@ hipError_t launch_stream_loads(const GemmArgs& g, int variant, int cus, int part
   const dim3 grid(stream_grid(g.N, cus)), block(kStream[variant].waves * 64);
   const int share = ceil_div(padded_n(g.N) / kNTile, (int)grid.x);
   int idx = 0;
-#define W4A8_STREAM_LOADS_GO(nt, kpw, w, p)                                                      \
-  if (parts == (p)) {                                                                            \
-    hipLaunchKernelGGL((gemm_stream_loads<nt, kpw, w, (p)>), grid, block, 0, stream, g.a,        \
-                       g.a_scale, g.wq, g.sq, out, g.M, g.K, g.N, share);                 \
+#define W4A8_STREAM_LOADS_GO(nt, kpw, w, p, tail)                                                \
+  if (parts == (p) && (g.K % kKAlign != 0) == (tail)) {                                          \
+    hipLaunchKernelGGL((gemm_stream_loads<nt, kpw, w, (p), (tail)>), grid, block, 0, stream,     \
+                       g.a, g.a_scale, g.wq, g.sq, out, g.M, g.K, g.N, share);                   \
     return hipGetLastError();                                                                    \
   }
 #define W4A8_STREAM_LOADS(nt, kpw, w)                                                            \
   if (idx++ == variant) {                                                                        \
-    W4A8_STREAM_LOADS_GO(nt, kpw, w, kStreamLoadWeights)                                         \
-    W4A8_STREAM_LOADS_GO(nt, kpw, w, kStreamLoadWeights | kStreamLoadScales)                     \
-    W4A8_STREAM_LOADS_GO(nt, kpw, w,                                                             \
-                         kStreamLoadWeights | kStreamLoadScales | kStreamLoadActivations)        \
+    W4A8_STREAM_LOADS_GO(nt, kpw, w, 1, false)                                                   \
+    W4A8_STREAM_LOADS_GO(nt, kpw, w, 3, false)                                                   \
+    W4A8_STREAM_LOADS_GO(nt, kpw, w, 7, false)                                                   \
+    W4A8_STREAM_LOADS_GO(nt, kpw, w, 1, true)                                                    \
+    W4A8_STREAM_LOADS_GO(nt, kpw, w, 3, true)                                                    \
+    W4A8_STREAM_LOADS_GO(nt, kpw, w, 7, true)                                                    \
     return hipErrorInvalidValue;                                                                 \
   }
   W4A8_STREAM_TABLE(W4A8_STREAM_LOADS)

@@ -149,7 +149,7 @@ int skinny_counter_count(int variant, int N);
 hipError_t launch_skinny(const GemmArgs& g, int variant, int split_k, float* partial,
                          int* counters, hipStream_t stream);
 
-// Streaming family (M <= 16, K % 512 == 0): grid = at most one workgroup per CU, each with the
+// Streaming family (M <= 16, K % 128 == 0): grid = at most one workgroup per CU, each with the
 // same number of n-tiles (at most nt); each of the `waves` waves owns a k-range of at most kpw
 // k-tiles across all of them (u = nt * kpw granules in registers). variant indexes the
 // instantiated table.
