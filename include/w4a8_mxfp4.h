@@ -110,7 +110,9 @@ int w4a8_gemm(const void* a, const float* a_scale, const void* wq, const void* s
  * its Python replica band_map (sly/mxfp4/band_map.py:31-95). For a macro-tile plan whose
  * workgroups fill a CU each, w4a8_gemm may run the variant on the leading columns that fill whole
  * rounds of workgroups and a 128 x 128 tile variant on the rest (two launches on the stream); the
- * returned triple names the first. A tile plan with split_k > 1 (the decode band's K split) is
+ * returned triple names the first. For 64 < M <= 1024 the triple names the plan's tile by its
+ * throughput table, and w4a8_gemm runs the macro tile that its time-per-slab table prices lowest
+ * (the same bits: a macro tile's shape does not change an output's accumulation order). A tile plan with split_k > 1 (the decode band's K split) is
  * two launches under w4a8_gemm_planned too: the partial launch and the reducing launch. */
 int w4a8_plan(int M, int N, int K, int* kernel, int* variant, int* split_k);
 

@@ -58,6 +58,8 @@ Scratch g_scratch[kMaxDevices];
 constexpr size_t kUnbounded = ~(size_t)0;
 // The automatic plan splits K across workgroups only in the decode band, M <= kMaxSplitM.
 constexpr int kMaxSplitM = 64;
+// Above the decode band and up to here the automatic path takes mid_tile_auto's tile.
+constexpr int kMidMaxM = 1024;
 const Scratch kPlanAnySplit{nullptr, kUnbounded, nullptr, kUnbounded, "unbounded scratch"};
 
 int current_device() {
@@ -205,6 +207,52 @@ int mid_tile(int M, int N, int cus) {
     const long per = ceil_div((long)ceil_div(M, c.bm) * ceil_div(N, c.bn), (long)cus);
     const double area = (double)c.bm * c.bn;
     const double cost = per == 2 ? 2 * area / t.r2 : per * area / t.r1;
+    if (pick < 0 || cost < best) best = cost, pick = v;
+  }
+  return pick;
+}
+
+// What the automatic path runs for 64 < M <= 1024: the tile with the least measured time per 128-k
+// slab, by the rounds of one tile per CU that the shape takes (1, 2 or 3; more in proportion to 3).
+// ns per slab on MI355X, medians over 8 decoder shapes (N 3584 .. 28672, K 3584 .. 9472) at M = 65,
+// 80, 96, 128, 160, 192, 200, 224, 256, 320, 384, 448, 512, 640, 768, 900 and 1024, weights
+// rotating through 400 MB, after 4 us of launch, first fill and epilogue. At these M a slab is
+// bound by LDS traffic (a 128 x 128 slab's fragment reads and fills take ~340 ns of LDS time against
+// ~215 ns of MFMA), so tiles whose waves own more columns per token row (a column is 64 bytes of a
+// slab, a token 128) and that read their fragments a slab ahead do best. Against the fastest tile at
+// each of the 136 points the pick is 0.4 % slower on average; against the throughput table above,
+// whose picks the plan names, it is 7 % faster (N = 17408 M = 200: 31.7 -> 27.5 us, N = 10240
+// M = 200 / 512: 21.4 -> 17.4, 32.7 -> 27.9, N = 5120 K = 8704 M = 200: 22.7 -> 18.9).
+struct TileSlab {
+  int wm, wn, nw, ns;
+  int t[3];
+};
+constexpr TileSlab kMidSlabs[] = {
+    {1, 3, 4, 8, {181, 389, 643}},      // 32 x 96
+    {2, 2, 4, 5, {197, 350, 608}},      // 64 x 64
+    {1, 4, 4, 8, {210, 460, 746}},      // 32 x 128
+    {2, 3, 4, 6, {250, 540, 856}},      // 64 x 96
+    {2, 4, 4, 4, {284, 566, 823}},      // 64 x 128
+    {2, 5, 4, 5, {328, 735, 1159}},     // 64 x 160
+    {3, 4, 4, 4, {329, 735, 1147}},     // 96 x 128
+    {2, 4, 8, 4, {389, 896, 1464}},     // 128 x 128
+    {2, 5, 8, 4, {468, 1106, 1737}},    // 128 x 160
+    {2, 6, 8, 4, {517, 1220, 1997}},    // 128 x 192
+    {4, 4, 8, 3, {628, 1510, 2438}},    // 256 x 128
+    {2, 8, 8, 4, {725, 1622, 2490}},    // 128 x 256
+    {4, 5, 8, 3, {790, 1858, 3124}},    // 256 x 160
+    {4, 8, 8, 3, {1133, 2599, 3900}},   // 256 x 256
+};
+
+int mid_tile_auto(int M, int N, int cus) {
+  double best = 0;
+  int pick = -1;
+  for (const TileSlab& s : kMidSlabs) {
+    const int v = find_tile(s.wm, s.wn, s.nw, s.ns);
+    if (v < 0) continue;
+    const TileCfg c = tile_variant(v);
+    const long rounds = ceil_div((long)ceil_div(M, c.bm) * ceil_div(N, c.bn), (long)cus);
+    const double cost = rounds <= 3 ? s.t[rounds - 1] : s.t[2] * (rounds / 3.0);
     if (pick < 0 || cost < best) best = cost, pick = v;
   }
   return pick;
@@ -371,7 +419,7 @@ int plan_tile(int M, int N, int dev) {
     if (tiles(64, 96) <= cus) return find_tile(1, 3, 8, 5);
     return find_tile(2, 4, 4, 4);
   }
-  if (M <= 1024) return mid_tile(M, N, cus);
+  if (M <= kMidMaxM) return mid_tile(M, N, cus);
   return big_tile(M, N, dev);
 }
 
@@ -521,6 +569,11 @@ int gemm_run(const void* a, const float* as, const void* wq, const void* sq, voi
       if (split_k == 1) variant = plan_tile(M, N, dev);
     } else {
       plan_impl(M, N, K, dev, sc, &kernel, &variant, &split_k);
+    }
+    if ((kernel == W4A8_KERNEL_TILE || kernel == W4A8_KERNEL_TILE_AT) && M > kMaxSplitM &&
+        M <= kMidMaxM && split_k <= 1) {
+      const int v = mid_tile_auto(M, N, device_info(dev).cus);
+      if (v >= 0) variant = v;
     }
     int tail = -1;
     const int n_main = (kernel == W4A8_KERNEL_TILE || kernel == W4A8_KERNEL_TILE_AT) &&

@@ -26,9 +26,19 @@
 //    ahead. The MFMA applies the scales, so no dequantisation happens anywhere.
 //  * Workgroups are renumbered so each XCD (hardware places workgroup b on XCD b % 8) gets a
 //    contiguous run of tiles, walked in groups of 8 row blocks, which keeps an XCD's activation
-//    and weight panels in its own L2.
+//    and weight panels in its own L2. Runs of unequal length where the tiles do not divide by 8
+//    (left in launch order they cost up to a third: N = 3584 K = 9472 M = 384 on 228 tiles of
+//    64 x 96 29.3 -> 23.3 us).
 //  * Epilogue: a lane holds 4 consecutive columns of one token; scaled by the per-token fp32 scale,
 //    rounded to bf16 and stored 8 bytes at a time.
+//  * AH = true reads every fragment one slab ahead, between the MFMAs of the slab before, so the
+//    LDS reads of a slab (64 KiB for 128 x 128 in 8 waves, ~250 ns) run under the MFMAs of the one
+//    before instead of in front of their own. Measured on MI355X (us, same bits): 128 x 128 in 8
+//    waves at N = 5120 K = 6144 M = 512 23.6 -> 22.0, N = 10240 M = 200 21.1 -> 19.9; 64 x 128 in 4
+//    waves at N = 5120 K = 6144 M = 200 16.7 -> 15.9; no gain up to 64 tokens, where the tiles are
+//    bound by their fills. The mid-M tiles use it (96 x 128, 64 x 96, 64 x 160 in 4 waves and
+//    128 x 128, 128 x 160, 128 x 192 in 8); the 256-row tiles keep the WM >= 3 pipeline, which needs
+//    fewer registers (256 x 256 ahead in 4 waves spilled 109 and took 734 us against 281).
 //  * AT = true reads the activations in the fragment-tiled layout the producers can write (16-token
 //    blocks of 16 x K bytes; in block b, k-tile t, half h, lane l's 16 bytes at
 //    ((b KT + t) 2 + h) 1024 + 16 l are token 16 b + l % 16, k-bytes 128 t + 16 (4 h + l / 16)):
@@ -120,7 +130,7 @@ static_assert(ring_slots_hold(), "scale ring: NS < 4 R - 6");
 // split_reduce adds them in split order, scales and rounds. A compile-time switch: the unsplit
 // kernels keep exactly their own code (a run-time k-range cost the 256 x 256 tile 20 spilled
 // registers and 28 % of its speed).
-template <int WM, int WN, int NS, int NW, bool AT, bool SPLIT>
+template <int WM, int WN, int NS, int NW, bool AH, bool AT, bool SPLIT>
 __device__ __forceinline__ void tile_body(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
     const uint32_t* __restrict__ Sq, uint16_t* __restrict__ C, int M, int N, int K, int KTp,
@@ -141,7 +151,9 @@ __device__ __forceinline__ void tile_body(
   constexpr unsigned GROUP = 8;
   const unsigned total = (unsigned)(grid_m * grid_n);
   unsigned t = blockIdx.x;
-  if ((total & 7) == 0) t = (t & 7) * (total >> 3) + (t >> 3);
+  // XCD x = t % 8 takes the run of total / 8 tiles (one more for the first total % 8 XCDs) that
+  // starts where XCD x - 1's ends
+  t = (t & 7) * (total >> 3) + min(t & 7, total & 7) + (t >> 3);
   unsigned bm = 0, bn = t;
   if (grid_m > 1) {
     const unsigned per_group = GROUP * (unsigned)grid_n;
@@ -282,7 +294,78 @@ __device__ __forceinline__ void tile_body(
   // every slab knows at compile time whether its refill carries a scale unit, and so how many
   // fills its wait may leave in flight.
 
-  if constexpr (WM >= 3) {
+  if constexpr (AH) {
+    // ---- NS-stage pipeline, every fragment one slab ahead: at the barrier of slab kt its
+    //      fragments are in registers (read during slab kt-1), every wave is done reading its stage
+    //      and slab kt+1's fills have landed; past it, the MFMAs of slab kt run from registers
+    //      while slab kt+1's fragment reads and the refill of slab kt's stage (slab kt+NS) go out
+    //      between them. ----
+#pragma unroll
+    for (int p = 0; p < NS; ++p) fill(kt0 + p, p);
+    wait_vmcnt<S::fills_after(0, NS - 1)>();     // the first slab and its scales have landed
+    bare_barrier();
+    v4i wf[WN], al[WM], ah[WM];
+    uint32_t sc[WN];
+    read_w(0, kt0, wf, sc);
+#pragma unroll
+    for (int i = 0; i < WM; ++i) read_a(0, i, al[i], ah[i]);
+    int st = 0;
+    auto slab = [&](int kt, auto qc) {
+      constexpr int q = decltype(qc)::value;    // kt % 4
+      constexpr int NF = S::fills(q + NS);       // fills of the refill, slab kt + NS
+      asm volatile("" : "+s"(kt));               // kt opaque: no per-copy loop invariants
+      const int nst = st + 1 == NS ? 0 : st + 1;
+      uint8_t* fbase = lds + st * S::STAGE;      // slab kt's stage, refilled with slab kt+NS
+      wait_vmcnt<S::fills_after(q + 1, NS - 2)>();  // this wave's fills of slab kt+1 landed
+      __builtin_amdgcn_s_waitcnt(0xC07F);        // lgkmcnt(0): this wave's reads of slab kt done
+      bare_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      const uint8_t* nbase = lds + nst * S::STAGE;
+      const uint8_t* srow = sring + (((kt + 1) >> 2) % RING) * S::S_SLOT + lane * 4;
+      v4i wfn[WN], aln[WM], ahn[WM];
+      uint32_t scn[WN];
+      // one memory step after each MFMA: the WN weight fragments, the WM activation fragments,
+      // then the refill's fills, spread over the slab's WM * WN MFMAs
+      constexpr int OPS_ALL = WN + WM + NF, MM = WM * WN;
+#pragma unroll
+      for (int m = 0; m < MM; ++m) {
+        const int i = m / WN, j = m % WN;
+        const v8i xf = {al[i][0], al[i][1], al[i][2], al[i][3],
+                        ah[i][0], ah[i][1], ah[i][2], ah[i][3]};
+        acc[i][j] = mfma_w4a8(wf[j], xf, acc[i][j], sc[j] >> (8 * q));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int o = m * OPS_ALL / MM; o < (m + 1) * OPS_ALL / MM; ++o) {
+          if (o < WN) {
+            wfn[o] = *reinterpret_cast<const v4i*>(nbase + S::W_OFF + (wn * WN + o) * 1024 +
+                                                   lane * 16);
+            // a k-group's scale dwords serve its 4 slabs: read them only for its first slab
+            if constexpr (q == 3)
+              scn[o] = *reinterpret_cast<const uint32_t*>(srow + (wn * WN + o) * 256);
+          } else if (o < WN + WM) {
+            read_a(nst, o - WN, aln[o - WN], ahn[o - WN]);
+          } else {
+            fill_any(kt + NS, fbase, o - WN - WM);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int j = 0; j < WN; ++j) {
+        wf[j] = wfn[j];
+        if constexpr (q == 3) sc[j] = scn[j];
+      }
+#pragma unroll
+      for (int i = 0; i < WM; ++i) al[i] = aln[i], ah[i] = ahn[i];
+      st = nst;
+    };
+    for (int kt = kt0; kt < kt1; kt += 4) {
+      slab(kt, IntC<0>{});
+      slab(kt + 1, IntC<1>{});
+      slab(kt + 2, IntC<2>{});
+      slab(kt + 3, IntC<3>{});
+    }
+  } else if constexpr (WM >= 3) {
     // ---- NS-stage pipeline, barrier two MFMA groups before the end of each slab. At the
     //      barrier of slab kt every wave has its own fills of slab kt+1 landed and has finished
     //      every read of slab kt; past it, the wave reads slab kt+1's weight fragments, scales
@@ -498,47 +581,49 @@ __device__ __forceinline__ void tile_body(
 // 32- and 64-token tiles of the decode band (4 waves), whose launches are short, measured
 // 0.15-0.25 us faster with it. The larger tiles keep the original order, with which their
 // register allocation spills least (the 8-wave 256 x 256 tile measured 8 % slower with the other).
-template <int WM, int WN, int NS, int NW, bool AT>
+template <int WM, int WN, int NS, int NW, bool AH, bool AT>
 __global__ __launch_bounds__(NW * 64) void gemm_tile(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
     const uint32_t* __restrict__ Sq, uint16_t* __restrict__ C, int M, int N, int K, int KTp,
     int KTe, int KG, int NTILES, int grid_m, int grid_n, int ldc, int vec_out) {
-  tile_body<WM, WN, NS, NW, AT, false>(A, As, Wq, Sq, C, M, N, K, KTp, KTe, KG, NTILES, grid_m,
+  tile_body<WM, WN, NS, NW, AH, AT, false>(A, As, Wq, Sq, C, M, N, K, KTp, KTe, KG, NTILES, grid_m,
                                        grid_n, ldc, vec_out, nullptr, 1);
 }
 
-template <int WM, int WN, int NS, int NW, bool AT>
+template <int WM, int WN, int NS, int NW, bool AH, bool AT>
 __global__ __launch_bounds__(NW * 64) void gemm_tile_pre(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
     const uint32_t* __restrict__ Sq, int M, int K, int KTp, int NTILES, int grid_m, int grid_n,
     int N, int ldc, int vec_out, uint16_t* __restrict__ C) {
-  tile_body<WM, WN, NS, NW, AT, false>(A, As, Wq, Sq, C, M, N, K, KTp, ceil_div(K, kKTile),
+  tile_body<WM, WN, NS, NW, AH, AT, false>(A, As, Wq, Sq, C, M, N, K, KTp, ceil_div(K, kKTile),
                                        KTp / kKGroup, NTILES, grid_m, grid_n, ldc, vec_out,
                                        nullptr, 1);
 }
 
 // The K-split form of the 4-wave band tiles (WM <= 2): the preloaded argument order of
 // gemm_tile_pre, then the partials and the split count.
-template <int WM, int WN, int NS, int NW, bool AT>
+template <int WM, int WN, int NS, int NW, bool AH, bool AT>
 __global__ __launch_bounds__(NW * 64) void gemm_tile_split(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
     const uint32_t* __restrict__ Sq, int M, int K, int KTp, int NTILES, int grid_m, int grid_n,
     int N, int splits, float* __restrict__ P) {
-  tile_body<WM, WN, NS, NW, AT, true>(A, As, Wq, Sq, nullptr, M, N, K, KTp, ceil_div(K, kKTile),
+  tile_body<WM, WN, NS, NW, AH, AT, true>(A, As, Wq, Sq, nullptr, M, N, K, KTp, ceil_div(K, kKTile),
                                       KTp / kKGroup, NTILES, grid_m, grid_n, N, 0, P, splits);
 }
 
 
-// (WM, WN, NS, NW): NW waves of 16 WM x 16 WN in an (NW / 2) x 2 arrangement, NS-stage LDS
-// pipeline (LDS = NS * STAGE + ring_slots(NS) scale slots + token scales <= 160 KiB)
+// (WM, WN, NS, NW, AH): NW waves of 16 WM x 16 WN in an (NW / 2) x 2 arrangement, NS-stage LDS
+// pipeline, AH 1 with every fragment read a slab ahead (LDS = NS * STAGE + ring_slots(NS) scale slots + token scales <= 160 KiB)
 #define W4A8_TILE_TABLE(X)                                                                        \
-  X(2, 4, 4, 4) X(4, 4, 3, 4) X(4, 4, 4, 4) X(8, 4, 3, 4) X(4, 8, 3, 4) X(8, 8, 3, 4)            \
-  X(8, 5, 3, 4) X(4, 8, 4, 4) X(4, 2, 4, 4) X(1, 2, 4, 4) X(2, 2, 4, 4) X(1, 4, 4, 4)            \
-  X(2, 2, 5, 4) X(4, 8, 3, 8) X(4, 5, 3, 8) X(2, 3, 4, 4) X(2, 1, 5, 4) X(1, 3, 4, 4)            \
-  X(1, 1, 5, 4) X(1, 1, 8, 4) X(1, 2, 8, 4) X(1, 3, 8, 4) X(1, 3, 5, 8) X(1, 4, 8, 4)            \
-  X(2, 4, 4, 8) X(2, 8, 4, 8) X(4, 4, 3, 8)
+  X(2, 4, 4, 4, 0) X(4, 4, 3, 4, 0) X(4, 4, 4, 4, 0) X(8, 4, 3, 4, 0) X(4, 8, 3, 4, 0)            \
+  X(8, 8, 3, 4, 0) X(8, 5, 3, 4, 0) X(4, 8, 4, 4, 0) X(4, 2, 4, 4, 0) X(1, 2, 4, 4, 0)            \
+  X(2, 2, 4, 4, 0) X(1, 4, 4, 4, 0) X(2, 2, 5, 4, 0) X(4, 8, 3, 8, 0) X(4, 5, 3, 8, 0)            \
+  X(2, 3, 4, 4, 0) X(2, 1, 5, 4, 0) X(1, 3, 4, 4, 0) X(1, 1, 5, 4, 0) X(1, 1, 8, 4, 0)            \
+  X(1, 2, 8, 4, 0) X(1, 3, 8, 4, 0) X(1, 3, 5, 8, 0) X(1, 4, 8, 4, 0) X(2, 4, 4, 8, 1)            \
+  X(2, 8, 4, 8, 0) X(4, 4, 3, 8, 0) X(2, 3, 6, 4, 1) X(2, 5, 5, 4, 1) X(3, 4, 4, 4, 1)            \
+  X(2, 5, 4, 8, 1) X(2, 6, 4, 8, 1)
 
-#define W4A8_TILE_CFG(wm, wn, ns, nw)                                                             \
+#define W4A8_TILE_CFG(wm, wn, ns, nw, ah)                                                          \
   TileCfg{wm, wn, TileShape<wm, wn, nw>::BM, TileShape<wm, wn, nw>::BN, nw,                        \
           ns * TileShape<wm, wn, nw>::STAGE + ring_slots(ns) * TileShape<wm, wn, nw>::S_SLOT +   \
               1024 +                                                                             \
@@ -618,30 +703,30 @@ hipError_t launch_tile_body(const GemmArgs& g, int variant, bool a_tiled, hipStr
                             float* P, int splits, int KTp, int KTe, int KG, int NTILES,
                             int grid_m, int grid_n, int vec_out, dim3 grid, dim3 block) {
   int idx = 0;
-#define W4A8_TILE_GO(wm, wn, ns, nw, at)                                                         \
+#define W4A8_TILE_GO(wm, wn, ns, nw, ah, at)                                                     \
   {                                                                                              \
     if (P) {                                                                                     \
       if constexpr (nw == 4 && wm <= 2)                                                          \
-        hipLaunchKernelGGL((gemm_tile_split<wm, wn, ns, nw, at>), grid, block, 0, stream, g.a,   \
-                           g.a_scale, g.wq, g.sq, g.M, g.K, KTp, NTILES, grid_m, grid_n, g.N,   \
-                           splits, P);                                                           \
+        hipLaunchKernelGGL((gemm_tile_split<wm, wn, ns, nw, ah, at>), grid, block, 0, stream,    \
+                           g.a, g.a_scale, g.wq, g.sq, g.M, g.K, KTp, NTILES, grid_m, grid_n,    \
+                           g.N, splits, P);                                                      \
       else                                                                                       \
         return hipErrorInvalidValue;                                                             \
     } else if constexpr (nw == 8 || wm > 2) {                                                    \
-      hipLaunchKernelGGL((gemm_tile<wm, wn, ns, nw, at>), grid, block, 0, stream, g.a,           \
+      hipLaunchKernelGGL((gemm_tile<wm, wn, ns, nw, ah, at>), grid, block, 0, stream, g.a,       \
                          g.a_scale, g.wq, g.sq, g.c, g.M, g.N, g.K, KTp, KTe, KG, NTILES, grid_m, \
                          grid_n, g.ldc, vec_out);                                                \
     } else {                                                                                     \
-      hipLaunchKernelGGL((gemm_tile_pre<wm, wn, ns, nw, at>), grid, block, 0, stream, g.a,       \
-                         g.a_scale, g.wq, g.sq, g.M, g.K, KTp, NTILES, grid_m, grid_n, g.N,     \
+      hipLaunchKernelGGL((gemm_tile_pre<wm, wn, ns, nw, ah, at>), grid, block, 0, stream, g.a,   \
+                         g.a_scale, g.wq, g.sq, g.M, g.K, KTp, NTILES, grid_m, grid_n, g.N,      \
                          g.ldc, vec_out, g.c);                                                   \
     }                                                                                            \
     return hipGetLastError();                                                                    \
   }
-#define W4A8_TILE_LAUNCH(wm, wn, ns, nw)                                                       \
+#define W4A8_TILE_LAUNCH(wm, wn, ns, nw, ah)                                                     \
   if (idx++ == variant) {                                                                        \
-    if (a_tiled) W4A8_TILE_GO(wm, wn, ns, nw, true)                                              \
-    W4A8_TILE_GO(wm, wn, ns, nw, false)                                                          \
+    if (a_tiled) W4A8_TILE_GO(wm, wn, ns, nw, ah != 0, true)                                     \
+    W4A8_TILE_GO(wm, wn, ns, nw, ah != 0, false)                                                 \
   }
   W4A8_TILE_TABLE(W4A8_TILE_LAUNCH)
 #undef W4A8_TILE_LAUNCH
