@@ -114,8 +114,7 @@ def _layout(q: torch.Tensor, M: int, K: int, tiled: bool) -> int:
 
 
 # ---- custom ops -------------------------------------------------------------------------------
-@torch.library.custom_op("radiance::add_rms_quant", mutates_args=())
-def add_rms_quant_op(y: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
+def _add_rms_quant(y: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
                      eps: float) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """y, residual: [M, K] bf16; weight: [K] bf16 (Gemma convention, the kernel adds the 1).
     Returns (q [M, K] e4m3, scale [M] f32, residual_out [M, K] bf16)
@@ -133,16 +132,19 @@ def add_rms_quant_op(y: torch.Tensor, residual: torch.Tensor, weight: torch.Tens
     return q, s, r
 
 
-@add_rms_quant_op.register_fake
-def _(y, residual, weight, eps):
+def _add_rms_quant_fake(y, residual, weight, eps):
     M, K = y.shape
     return (torch.empty((M, K), device=y.device, dtype=torch.float8_e4m3fn),
             torch.empty((M,), device=y.device, dtype=torch.float32),
             torch.empty((M, K), device=y.device, dtype=torch.bfloat16))
 
 
-@torch.library.custom_op("radiance::silu_mul_quant", mutates_args=())
-def silu_mul_quant_op(gate_up: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+add_rms_quant_op = torch.library.custom_op("radiance::add_rms_quant", _add_rms_quant, mutates_args=())
+add_rms_quant_op.register_fake(_add_rms_quant_fake)
+call_add_rms_quant = _rmx.inference_op(add_rms_quant_op, _add_rms_quant, _add_rms_quant_fake)
+
+
+def _silu_mul_quant(gate_up: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """gate_up: [M, 2N] bf16 -> (q [M, N] e4m3 of silu(gate) * up, scale [M] f32)
     (sly/mxfp4/radiance_fused_norm.py:163-180)."""
     _need_bf16("silu_mul_quant", gate_up=gate_up)
@@ -157,15 +159,18 @@ def silu_mul_quant_op(gate_up: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor
     return q, s
 
 
-@silu_mul_quant_op.register_fake
-def _(gate_up):
+def _silu_mul_quant_fake(gate_up):
     M, N2 = gate_up.shape
     return (torch.empty((M, N2 // 2), device=gate_up.device, dtype=torch.float8_e4m3fn),
             torch.empty((M,), device=gate_up.device, dtype=torch.float32))
 
 
-@torch.library.custom_op("radiance::gdn_norm_quant", mutates_args=())
-def gdn_norm_quant_op(x: torch.Tensor, z: torch.Tensor, weight: torch.Tensor,
+silu_mul_quant_op = torch.library.custom_op("radiance::silu_mul_quant", _silu_mul_quant, mutates_args=())
+silu_mul_quant_op.register_fake(_silu_mul_quant_fake)
+call_silu_mul_quant = _rmx.inference_op(silu_mul_quant_op, _silu_mul_quant, _silu_mul_quant_fake)
+
+
+def _gdn_norm_quant(x: torch.Tensor, z: torch.Tensor, weight: torch.Tensor,
                       eps: float) -> tuple[torch.Tensor, torch.Tensor]:
     """x: [M, N] bf16 (N = heads * 128); z: [M, N] bf16, any row stride as long as each row is a
     contiguous run; weight: [128] bf16. Returns (q [M, N] e4m3, scale [M] f32)
@@ -183,11 +188,15 @@ def gdn_norm_quant_op(x: torch.Tensor, z: torch.Tensor, weight: torch.Tensor,
     return q, s
 
 
-@gdn_norm_quant_op.register_fake
-def _(x, z, weight, eps):
+def _gdn_norm_quant_fake(x, z, weight, eps):
     M, N = x.shape
     return (torch.empty((M, N), device=x.device, dtype=torch.float8_e4m3fn),
             torch.empty((M,), device=x.device, dtype=torch.float32))
+
+
+gdn_norm_quant_op = torch.library.custom_op("radiance::gdn_norm_quant", _gdn_norm_quant, mutates_args=())
+gdn_norm_quant_op.register_fake(_gdn_norm_quant_fake)
+call_gdn_norm_quant = _rmx.inference_op(gdn_norm_quant_op, _gdn_norm_quant, _gdn_norm_quant_fake)
 
 
 # ---- where a fusion is valid ------------------------------------------------------------------
@@ -358,14 +367,14 @@ def gdn_ok(attn) -> bool:
 # ---- call-site helpers (names and signatures the model patch calls) -----------------------------
 def add_rms_quant(norm, hidden_states: torch.Tensor, residual: torch.Tensor):
     """Stands in for norm(hidden_states, residual): returns ((q, scale), new residual)."""
-    q, scale, new_residual = torch.ops.radiance.add_rms_quant(
+    q, scale, new_residual = call_add_rms_quant(
         hidden_states, residual, norm.weight, norm.variance_epsilon)
     return (q, scale), new_residual
 
 
 def silu_mul_quant(gate_up: torch.Tensor):
     """Stands in for act_fn(gate_up): returns (q, scale)."""
-    return tuple(torch.ops.radiance.silu_mul_quant(gate_up))
+    return tuple(call_silu_mul_quant(gate_up))
 
 
 def silu_mul_down(down, gate_up: torch.Tensor):
@@ -378,7 +387,7 @@ def silu_mul_down(down, gate_up: torch.Tensor):
     layer has skip_bias_add (then output_bias is the bias, else None), or output alone when the
     layer has return_bias = False."""
     lead = gate_up.shape[:-1]
-    y = torch.ops.radiance.silu_mul_mxfp4_linear(gate_up.reshape(-1, gate_up.shape[-1]),
+    y = _rmx.call_silu_mul_linear(gate_up.reshape(-1, gate_up.shape[-1]),
                                                  down.weight, down.weight_scale,
                                                  down.radiance_wref)
     bias = getattr(down, "bias", None)
@@ -394,5 +403,5 @@ def silu_mul_down(down, gate_up: torch.Tensor):
 def gdn_norm_quant(attn, core_attn_out: torch.Tensor, z: torch.Tensor):
     """Stands in for attn.norm(core_attn_out, z) flattened to one row per token: (q, scale)."""
     tokens = core_attn_out.shape[0]
-    return tuple(torch.ops.radiance.gdn_norm_quant(
+    return tuple(call_gdn_norm_quant(
         core_attn_out.reshape(tokens, -1), z.reshape(tokens, -1), attn.norm.weight, attn.norm.eps))

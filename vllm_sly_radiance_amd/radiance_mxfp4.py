@@ -206,8 +206,32 @@ def gemm(x_fp8: torch.Tensor, x_scale: torch.Tensor, weight: torch.Tensor,
 # --------------------------------------------------------------------------------------------
 # Custom ops: the whole path is one opaque node (sly/mxfp4/radiance_mxfp4.py:644-652)
 # --------------------------------------------------------------------------------------------
-@torch.library.custom_op("radiance::mxfp4_linear", mutates_args=())
-def mxfp4_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor,
+_fragment = torch.library.Library("radiance", "FRAGMENT")
+
+
+def inference_op(op, body, fake):
+    """A second registration of the custom op `op`, radiance::<name>_inference: the same schema and
+    body straight on the dispatcher, without custom_op's Python autograd and alias-checking layers.
+    Those take ~9.5 of the ~14 us a custom_op call costs before its body, more than the GPU time of a
+    small linear (one token through N = 10240 K = 5120, called from Python: 21 us a call, 6 of them
+    on the GPU). Returns a callable that takes the second form where no gradient can be asked for
+    and nothing is being compiled, and `op` (whose backward raises) otherwise."""
+    ns, name = op._qualname.split("::")
+    schema = str(op._opoverload._schema)
+    _fragment.define(schema.replace(f"{ns}::{name}(", f"{name}_inference(", 1))
+    _fragment.impl(f"{name}_inference", body, "CompositeExplicitAutograd")
+    torch.library.register_fake(f"{ns}::{name}_inference", fake)
+    public, direct = op._opoverload, getattr(torch.ops.radiance, f"{name}_inference").default
+
+    def call(*args):
+        if torch.compiler.is_compiling() or (torch.is_grad_enabled() and any(
+                a.requires_grad for a in args if isinstance(a, torch.Tensor))):
+            return public(*args)
+        return direct(*args)
+    return call
+
+
+def _mxfp4_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor,
                  weight_ref: torch.Tensor) -> torch.Tensor:
     """bf16 x [M, K] -> bf16 [M, N]: per-token e4m3 quant + W4A8 GEMM on the current stream. At
     M <= 2 (M <= 4 where the plan leaves its quantizing waves little work) one launch quantizes
@@ -235,13 +259,16 @@ def mxfp4_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tens
     return _diag.returned(out)
 
 
-@mxfp4_linear.register_fake
-def _(x, weight, weight_scale, weight_ref):
+def _mxfp4_linear_fake(x, weight, weight_scale, weight_ref):
     return torch.empty((x.shape[0], weight_ref.shape[0]), device=x.device, dtype=torch.bfloat16)
 
 
-@torch.library.custom_op("radiance::mxfp4_linear_pq", mutates_args=())
-def mxfp4_linear_pq(x_fp8: torch.Tensor, x_scale: torch.Tensor, weight: torch.Tensor,
+mxfp4_linear = torch.library.custom_op("radiance::mxfp4_linear", _mxfp4_linear, mutates_args=())
+mxfp4_linear.register_fake(_mxfp4_linear_fake)
+call_linear = inference_op(mxfp4_linear, _mxfp4_linear, _mxfp4_linear_fake)
+
+
+def _mxfp4_linear_pq(x_fp8: torch.Tensor, x_scale: torch.Tensor, weight: torch.Tensor,
                     weight_scale: torch.Tensor, weight_ref: torch.Tensor,
                     allow_tiled: bool = True) -> torch.Tensor:
     """Pre-quantized entry (sly/mxfp4/radiance_mxfp4.py:825-860): (e4m3 [M, K], fp32 [M]) -> bf16
@@ -272,14 +299,18 @@ def mxfp4_linear_pq(x_fp8: torch.Tensor, x_scale: torch.Tensor, weight: torch.Te
     return _diag.returned(out)
 
 
-@mxfp4_linear_pq.register_fake
-def _(x_fp8, x_scale, weight, weight_scale, weight_ref, allow_tiled=True):
+def _mxfp4_linear_pq_fake(x_fp8, x_scale, weight, weight_scale, weight_ref, allow_tiled=True):
     return torch.empty((x_fp8.shape[0], weight_ref.shape[0]), device=x_fp8.device,
                        dtype=torch.bfloat16)
 
 
-@torch.library.custom_op("radiance::silu_mul_mxfp4_linear", mutates_args=())
-def silu_mul_mxfp4_linear(gate_up: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor,
+mxfp4_linear_pq = torch.library.custom_op("radiance::mxfp4_linear_pq", _mxfp4_linear_pq,
+                                          mutates_args=())
+mxfp4_linear_pq.register_fake(_mxfp4_linear_pq_fake)
+call_linear_pq = inference_op(mxfp4_linear_pq, _mxfp4_linear_pq, _mxfp4_linear_pq_fake)
+
+
+def _silu_mul_mxfp4_linear(gate_up: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor,
                           weight_ref: torch.Tensor) -> torch.Tensor:
     """The MLP's tail in one op: gate_up bf16 [M, 2K] -> the down projection [M, N] of
     silu(gate) * up, the same bits as radiance::silu_mul_quant followed by mxfp4_linear_pq (the
@@ -314,10 +345,16 @@ def silu_mul_mxfp4_linear(gate_up: torch.Tensor, weight: torch.Tensor, weight_sc
     return _diag.returned(out)
 
 
-@silu_mul_mxfp4_linear.register_fake
-def _(gate_up, weight, weight_scale, weight_ref):
+def _silu_mul_mxfp4_linear_fake(gate_up, weight, weight_scale, weight_ref):
     return torch.empty((gate_up.shape[0], weight_ref.shape[0]), device=gate_up.device,
                        dtype=torch.bfloat16)
+
+
+silu_mul_mxfp4_linear = torch.library.custom_op(
+    "radiance::silu_mul_mxfp4_linear", _silu_mul_mxfp4_linear, mutates_args=())
+silu_mul_mxfp4_linear.register_fake(_silu_mul_mxfp4_linear_fake)
+call_silu_mul_linear = inference_op(silu_mul_mxfp4_linear, _silu_mul_mxfp4_linear,
+                                    _silu_mul_mxfp4_linear_fake)
 
 
 # --------------------------------------------------------------------------------------------
@@ -430,11 +467,11 @@ def _make_kernel_class():
         def apply_weights(self, layer: torch.nn.Module, x, bias: torch.Tensor | None = None):
             if isinstance(x, tuple):
                 x_fp8, x_scale = x
-                y = torch.ops.radiance.mxfp4_linear_pq(
+                y = call_linear_pq(
                     x_fp8, x_scale, layer.weight, layer.weight_scale, layer.radiance_wref)
             else:
                 lead = x.shape[:-1]
-                y = torch.ops.radiance.mxfp4_linear(
+                y = call_linear(
                     x.reshape(-1, x.shape[-1]), layer.weight, layer.weight_scale,
                     layer.radiance_wref)
                 y = y.reshape(*lead, y.shape[-1])
