@@ -208,6 +208,11 @@ int w4a8_workspace_bytes(int max_m, int max_n, size_t* partial_bytes, size_t* co
 int w4a8_linear(const void* x, long ldx, void* q, float* scale, const void* wq, const void* sq,
                 void* c, int M, int N, int K, void* stream);
 
+/* w4a8_linear with a bf16 bias [N] (16-byte aligned) added to the rounded outputs in the GEMM's
+ * epilogue: the bits of w4a8_linear followed by an elementwise bf16 add. */
+int w4a8_linear_bias(const void* x, long ldx, void* q, float* scale, const void* wq, const void* sq,
+                     const void* bias, void* c, int M, int N, int K, void* stream);
+
 /* 1 when w4a8_linear runs this shape (with a 16-byte aligned x) as one launch, 0 when as the
  * quantizer and the GEMM, -1 for a bad shape. No counterpart in the reference, whose op always
  * quantizes in a separate launch. */

@@ -46,6 +46,7 @@ SIGNATURES = {
     "w4a8_scratch_bytes": (_int, [_int, _int, _int, _psz, _psz]),
     "w4a8_workspace_bytes": (_int, [_int, _int, _psz, _psz]),
     "w4a8_linear": (_int, [_vp, _long, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp]),
+    "w4a8_linear_bias": (_int, [_vp, _long, _vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp]),
     "w4a8_linear_fused": (_int, [_int, _int, _int, _long]),
     "w4a8_add_rms_quant": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _int, _int, _c.c_float, _vp,
                                   _int]),
@@ -139,8 +140,12 @@ def tiled_bytes(M: int, K: int) -> int:
     return n.value
 
 
-def linear(x_ptr, ldx, q_ptr, s_ptr, wq_ptr, sq_ptr, c_ptr, M, N, K, stream):
-    check(lib().w4a8_linear(x_ptr, ldx, q_ptr, s_ptr, wq_ptr, sq_ptr, c_ptr, M, N, K, stream))
+def linear(x_ptr, ldx, q_ptr, s_ptr, wq_ptr, sq_ptr, c_ptr, M, N, K, stream, bias_ptr=0):
+    if bias_ptr:
+        check(lib().w4a8_linear_bias(x_ptr, ldx, q_ptr, s_ptr, wq_ptr, sq_ptr, bias_ptr, c_ptr, M,
+                                     N, K, stream))
+    else:
+        check(lib().w4a8_linear(x_ptr, ldx, q_ptr, s_ptr, wq_ptr, sq_ptr, c_ptr, M, N, K, stream))
 
 
 def linear_fused(M: int, N: int, K: int, ldx: int) -> bool:

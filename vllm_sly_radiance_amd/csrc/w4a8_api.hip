@@ -449,19 +449,19 @@ int tile_split(int M, int N, int variant, int dev, int* tail_variant) {
 // output are offset by n0 / 16 n-tiles; the output keeps its row stride N.
 int tile_columns(const void* a, const float* as, const void* wq, const void* sq, void* c, int M,
                  int N, int K, int n0, int n, int variant, bool a_tiled, const char* who,
-                 hipStream_t st) {
+                 hipStream_t st, const uint16_t* bias) {
   const size_t kt = padded_k(K) / kKTile, nt0 = n0 / kNTile;
   const GemmArgs g{(const uint8_t*)a, as, (const uint8_t*)wq + nt0 * kt * kGranuleBytes,
                    (const uint32_t*)sq + nt0 * (kt / kKGroup) * 64, (uint16_t*)c + n0, M, n, K,
-                   N};
+                   N, bias ? bias + n0 : nullptr};
   return hip_status(launch_tile(g, variant, a_tiled, st), who);
 }
 
 int gemm_dispatch(const void* a, const float* as, const void* wq, const void* sq, void* c, int M,
                   int N, int K, int kernel, int variant, int split_k, const Scratch& sc,
-                  const char* who, void* stream) {
+                  const char* who, void* stream, const uint16_t* bias) {
   const GemmArgs g{(const uint8_t*)a, as, (const uint8_t*)wq, (const uint32_t*)sq, (uint16_t*)c,
-                   M, N, K, N};
+                   M, N, K, N, bias};
   const hipStream_t st = (hipStream_t)stream;
   if (kernel == W4A8_KERNEL_SKINNY) {
     if (variant < 0 || variant >= skinny_variant_count())
@@ -549,7 +549,7 @@ int gemm_dispatch(const void* a, const float* as, const void* wq, const void* sq
 // which the tile kernel alone reads (the automatic plan is then plan_tile's).
 int gemm_run(const void* a, const float* as, const void* wq, const void* sq, void* c, int M, int N,
              int K, int kernel, int variant, int split_k, bool a_tiled, const Scratch& sc,
-             const char* who, void* stream) {
+             const char* who, void* stream, const uint16_t* bias = nullptr) {
   if (int e = check_gemm_shape(who, M, N, K)) return e;
   a_tiled = a_tiled || kernel == W4A8_KERNEL_TILE_AT || kernel == W4A8_KERNEL_RING_AT;
   if (a_tiled && kernel != W4A8_KERNEL_AUTO && kernel != W4A8_KERNEL_TILE_AT &&
@@ -582,12 +582,14 @@ int gemm_run(const void* a, const float* as, const void* wq, const void* sq, voi
                            : 0;
     if (n_main > 0 && n_main < N && n_main % kNTile == 0) {
       const hipStream_t st = (hipStream_t)stream;
-      if (int e = tile_columns(a, as, wq, sq, c, M, N, K, 0, n_main, variant, a_tiled, who, st))
+      if (int e = tile_columns(a, as, wq, sq, c, M, N, K, 0, n_main, variant, a_tiled, who, st,
+                               bias))
         return e;
-      return tile_columns(a, as, wq, sq, c, M, N, K, n_main, N - n_main, tail, a_tiled, who, st);
+      return tile_columns(a, as, wq, sq, c, M, N, K, n_main, N - n_main, tail, a_tiled, who, st,
+                          bias);
     }
   }
-  return gemm_dispatch(a, as, wq, sq, c, M, N, K, kernel, variant, split_k, sc, who, stream);
+  return gemm_dispatch(a, as, wq, sq, c, M, N, K, kernel, variant, split_k, sc, who, stream, bias);
 }
 
 }  // namespace
@@ -861,23 +863,39 @@ W4A8_API int w4a8_linear_fused(int M, int N, int K, long ldx) {
   return linear_fused_variant(M, N, K, ldx, true, current_device()) >= 0 ? 1 : 0;
 }
 
-W4A8_API int w4a8_linear(const void* x, long ldx, void* q, float* scale, const void* wq,
-                         const void* sq, void* c, int M, int N, int K, void* stream) {
-  if (int e = check_gemm_shape("w4a8_linear", M, N, K)) return e;
+static int linear_run(const char* who, const void* x, long ldx, void* q, float* scale,
+                      const void* wq, const void* sq, const uint16_t* bias, void* c, int M, int N,
+                      int K, void* stream) {
+  if (int e = check_gemm_shape(who, M, N, K)) return e;
   if (M == 0) return W4A8_OK;
-  if (int e = check_gemm_ptrs("w4a8_linear", q, scale, wq, sq, c)) return e;
-  if (!x) return fail(W4A8_EINVAL, "w4a8_linear: null x");
-  if (ldx < K) return fail(W4A8_EINVAL, "w4a8_linear: ldx=%ld < K=%d", ldx, K);
+  if (int e = check_gemm_ptrs(who, q, scale, wq, sq, c)) return e;
+  if (!x) return fail(W4A8_EINVAL, "%s: null x", who);
+  if (ldx < K) return fail(W4A8_EINVAL, "%s: ldx=%ld < K=%d", who, ldx, K);
   const int dev = current_device();
   const int v = linear_fused_variant(M, N, K, ldx, aligned(x, 16), dev);
   if (v >= 0) {
     const GemmArgs g{(const uint8_t*)x, nullptr, (const uint8_t*)wq, (const uint32_t*)sq,
-                     (uint16_t*)c, M, N, K, N};
+                     (uint16_t*)c, M, N, K, N, bias};
     return hip_status(launch_stream(g, v, device_info(dev).cus, true, ldx, (hipStream_t)stream),
-                      "w4a8_linear");
+                      who);
   }
   if (int e = w4a8_quant_per_token(x, ldx, q, scale, M, K, stream)) return e;
-  return w4a8_gemm(q, scale, wq, sq, c, M, N, K, stream);
+  return gemm_run(q, scale, wq, sq, c, M, N, K, W4A8_KERNEL_AUTO, -1, 0, false,
+                  registered_scratch(dev), who, stream, bias);
+}
+
+W4A8_API int w4a8_linear(const void* x, long ldx, void* q, float* scale, const void* wq,
+                         const void* sq, void* c, int M, int N, int K, void* stream) {
+  return linear_run("w4a8_linear", x, ldx, q, scale, wq, sq, nullptr, c, M, N, K, stream);
+}
+
+W4A8_API int w4a8_linear_bias(const void* x, long ldx, void* q, float* scale, const void* wq,
+                              const void* sq, const void* bias, void* c, int M, int N, int K,
+                              void* stream) {
+  if (!bias || !aligned(bias, 16))
+    return fail(W4A8_EINVAL, "w4a8_linear_bias: bias must be 16-byte aligned and not null");
+  return linear_run("w4a8_linear_bias", x, ldx, q, scale, wq, sq, (const uint16_t*)bias, c, M, N, K,
+                    stream);
 }
 
 // q_layout: W4A8_Q_ROWS, or W4A8_Q_TILED when the row length is whole 128-byte k-tiles

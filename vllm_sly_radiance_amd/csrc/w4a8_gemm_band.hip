@@ -92,7 +92,8 @@ __device__ __forceinline__ void band_post(int* counter, int v) {
 template <int MF, int NT, int SG, int R, int D, int L>
 __device__ __forceinline__ void band_body(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
-    const uint32_t* __restrict__ Sq, void* __restrict__ out, int mks, int K, int N, int S) {
+    const uint32_t* __restrict__ Sq, void* __restrict__ out, int mks, int K, int N, int S,
+    const uint16_t* __restrict__ bias) {
   static_assert(MF >= 1 && MF <= 4 && NT >= 1 && SG >= 2 && R >= 1, "band variant");
   static_assert(L >= 1 && L <= D && (L - 1) * 2 * MF < 64, "an activation wave may not run past "
                 "the slots it owns, and its loads in flight fit the load counter");
@@ -275,23 +276,23 @@ __device__ __forceinline__ void band_body(
       const float sc = tsc[m];
       uint16_t* const row = reinterpret_cast<uint16_t*>(out) + (size_t)m * N;
       if (N % 4 == 0 && ((uintptr_t)out & 7) == 0 && n + 3 < N) {
-        *reinterpret_cast<uint2*>(row + n) =
-            make_uint2(bf16x2_rne(v[0] * sc, v[1] * sc), bf16x2_rne(v[2] * sc, v[3] * sc));
+        uint2 y = make_uint2(bf16x2_rne(v[0] * sc, v[1] * sc), bf16x2_rne(v[2] * sc, v[3] * sc));
+        if (bias) y = add_bias4(y, bias, n, N);
+        *reinterpret_cast<uint2*>(row + n) = y;
       } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (n + i < N) row[n + i] = (uint16_t)f32_to_bf16(v[i] * sc);
+        store_out4(reinterpret_cast<uint16_t*>(out), N, m, n, N, v, sc, false, bias);
       }
     }
   }
 }
 
-// The 14 argument dwords are the preloaded ones.
+// The first 14 argument dwords are the preloaded ones; the bias is read in the epilogue.
 template <int MF, int NT, int SG, int R, int D, int L>
 __global__ __launch_bounds__(2 * kBandWW * 64) void gemm_band(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
-    const uint32_t* __restrict__ Sq, void* __restrict__ out, int mks, int K, int N, int S) {
-  band_body<MF, NT, SG, R, D, L>(A, As, Wq, Sq, out, mks, K, N, S);
+    const uint32_t* __restrict__ Sq, void* __restrict__ out, int mks, int K, int N, int S,
+    const uint16_t* __restrict__ bias) {
+  band_body<MF, NT, SG, R, D, L>(A, As, Wq, Sq, out, mks, K, N, S, bias);
 }
 
 // (MF, NT, SG, R, D, L): MF 16-token fragments, at most NT n-tiles per workgroup, SG scale dwords
@@ -371,7 +372,8 @@ hipError_t launch_band(const GemmArgs& g, int variant, int cus, int splits, floa
       if (e != hipSuccess) return e;                                                             \
     }                                                                                            \
     hipLaunchKernelGGL((gemm_band<mf, nt, sg, r, d, l>), dim3(G, rows), dim3(2 * kBandWW * 64),  \
-                       lds, stream, g.a, g.a_scale, g.wq, g.sq, out, mks, g.K, g.N, share);     \
+                       lds, stream, g.a, g.a_scale, g.wq, g.sq, out, mks, g.K, g.N, share,      \
+                       g.bias);                                                                 \
     const hipError_t e = hipGetLastError();                                                      \
     if (e != hipSuccess || splits <= 1) return e;                                                \
     return launch_split_reduce(partial, g, rows, stream);                                        \

@@ -25,7 +25,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
     const uint32_t* __restrict__ Sq, uint16_t* __restrict__ C, float* __restrict__ P,
     int* __restrict__ cnt, int M, int N, int K, int KTp, int KTe, int KG, int NTILES,
-    int kt_per_split, int vec_out) {
+    int kt_per_split, int vec_out, const uint16_t* __restrict__ bias) {
   constexpr int SLOTS = MT * NT * 64;   // one v4f (4 outputs) per slot
   constexpr int NTHR = WAVES * 64;
   __shared__ v4f red[WAVES > 1 ? WAVES * SLOTS : 1];
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny(
     const int p = slot >> 6, l = slot & 63;
     const int m = (p / NT) * 16 + (l & 15);
     const int n = (nt0 + p % NT) * kNTile + 4 * (l >> 4);
-    if (m < M) store_out4(C, N, m, n, N, v, As[m], vec_out != 0);
+    if (m < M) store_out4(C, N, m, n, N, v, As[m], vec_out != 0, bias);
   };
 
   if constexpr (WAVES > 1) {
@@ -181,7 +181,7 @@ hipError_t launch_skinny(const GemmArgs& g, int variant, int split_k, float* par
   if (idx++ == variant) {                                                                        \
     hipLaunchKernelGGL((gemm_skinny<mt, nt, w, u>), grid, block, 0, stream, g.a, g.a_scale,      \
                        g.wq, g.sq, g.c, partial, counters, g.M, g.N, g.K, KTp, KTe, KG, NTILES,  \
-                       per, vec_out);                                                            \
+                       per, vec_out, g.bias);                                                    \
     return hipGetLastError();                                                                    \
   }
   W4A8_SKINNY_TABLE(W4A8_SKINNY_LAUNCH)

@@ -66,13 +66,14 @@ __device__ __forceinline__ void lds_barrier() {
 // live tokens (lanes 8..15 of each row of 16 load the second run of token r - 8, and a row
 // rotation by 8 lanes hands it to lane r), half the activation loads; the MFMA columns of tokens
 // 8..15 then hold other tokens' bytes, and those columns are never stored.
-// The 14 argument dwords are exactly what the kernel arguments preloaded into SGPRs hold, so no
+// The first 14 argument dwords (all but the bias, which BIAS alone reads) are exactly what the kernel arguments preloaded into SGPRs hold, so no
 // wave reads the kernarg segment, not even for the epilogue (whose scalar load used to sit on the
 // critical path after the last MFMA); the n-tile count and the store width follow from N and C.
-template <int NT, int KPW, int W, bool H8, bool TAIL>
+template <int NT, int KPW, int W, bool H8, bool TAIL, bool BIAS>
 __global__ __launch_bounds__(W * 64) void gemm_stream(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
-    const uint32_t* __restrict__ Sq, uint16_t* __restrict__ C, int M, int K, int N, int S) {
+    const uint32_t* __restrict__ Sq, uint16_t* __restrict__ C, int M, int K, int N, int S,
+    const uint16_t* __restrict__ bias) {
   static_assert(KPW % 4 == 0 && NT >= 1 && W >= 1 && W <= 16, "stream variant");
   // K % 128 == 0; K, N > 0 (unsigned shifts: no sign fix-ups in the scalar prologue). KT
   // activation k-tiles; the weights are padded to KTP, whole k-groups, with zeros.
@@ -233,12 +234,12 @@ __global__ __launch_bounds__(W * 64) void gemm_stream(
     const int n = (ntb0 + t) * kNTile + 4 * og;
     uint16_t* row = C + (size_t)om * N;
     if (N % 4 == 0 && ((uintptr_t)C & 7) == 0 && n + 3 < N) {
-      *reinterpret_cast<uint2*>(row + n) = make_uint2(bf16x2_rne(v[0] * tok_scale, v[1] * tok_scale),
-                                                      bf16x2_rne(v[2] * tok_scale, v[3] * tok_scale));
+      uint2 y = make_uint2(bf16x2_rne(v[0] * tok_scale, v[1] * tok_scale),
+                           bf16x2_rne(v[2] * tok_scale, v[3] * tok_scale));
+      if constexpr (BIAS) y = add_bias4(y, bias, n, N);
+      *reinterpret_cast<uint2*>(row + n) = y;
     } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (n + i < N) row[n + i] = (uint16_t)f32_to_bf16(v[i] * tok_scale);
+      store_out4(C, N, om, n, N, v, tok_scale, false, BIAS ? bias : nullptr);
     }
   }
 }
@@ -397,10 +398,11 @@ __device__ __forceinline__ void fq_signal(int* counter) {
     __hip_atomic_fetch_add(counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-template <int NT, int KPW, int W, bool SILU, bool TAIL>
+template <int NT, int KPW, int W, bool SILU, bool TAIL, bool BIAS>
 __global__ __launch_bounds__(kFqWaves * 64) void gemm_stream_fq(
     const uint8_t* __restrict__ X, const uint8_t* __restrict__ Wq, const uint32_t* __restrict__ Sq,
-    uint16_t* __restrict__ C, int M, int K, int N, int S, int ldx) {
+    uint16_t* __restrict__ C, int M, int K, int N, int S, int ldx,
+    const uint16_t* __restrict__ bias) {
   constexpr int Q = kFqWaves - W;                // quantizing waves
   static_assert(KPW % 4 == 0 && NT >= 1 && W >= 1 && Q >= 4 && Q <= 12, "fq variant");
   // K % 128 == 0; K, N > 0 (unsigned shifts: no sign fix-ups in the scalar prologue). KT
@@ -574,12 +576,12 @@ __global__ __launch_bounds__(kFqWaves * 64) void gemm_stream_fq(
     const int n = (ntb0 + t) * kNTile + 4 * (c >> 3);
     uint16_t* row = C + (size_t)om * N;
     if (N % 4 == 0 && ((uintptr_t)C & 7) == 0 && n + 3 < N) {
-      *reinterpret_cast<uint2*>(row + n) = make_uint2(bf16x2_rne(v[0] * tok_scale, v[1] * tok_scale),
-                                                      bf16x2_rne(v[2] * tok_scale, v[3] * tok_scale));
+      uint2 y = make_uint2(bf16x2_rne(v[0] * tok_scale, v[1] * tok_scale),
+                           bf16x2_rne(v[2] * tok_scale, v[3] * tok_scale));
+      if constexpr (BIAS) y = add_bias4(y, bias, n, N);
+      *reinterpret_cast<uint2*>(row + n) = y;
     } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (n + i < N) row[n + i] = (uint16_t)f32_to_bf16(v[i] * tok_scale);
+      store_out4(C, N, om, n, N, v, tok_scale, false, BIAS ? bias : nullptr);
     }
   }
 }
@@ -676,39 +678,44 @@ hipError_t launch_stream(const GemmArgs& g, int variant, int cus, bool fused, lo
                                              (int)lds);                                          \
     if (e != hipSuccess) return e;                                                               \
   }
-#define W4A8_STREAM_GO(nt, kpw, w, h8, tail)                                                     \
+#define W4A8_STREAM_GO(nt, kpw, w, h8, tail, wb)                                                \
   {                                                                                              \
-    W4A8_STREAM_ATTR((gemm_stream<nt, kpw, w, h8, tail>))                                        \
-    hipLaunchKernelGGL((gemm_stream<nt, kpw, w, h8, tail>), grid, block, lds, stream, g.a,       \
-                       g.a_scale, g.wq, g.sq, g.c, g.M, g.K, g.N, share);                        \
+    W4A8_STREAM_ATTR((gemm_stream<nt, kpw, w, h8, tail, wb>))                                  \
+    hipLaunchKernelGGL((gemm_stream<nt, kpw, w, h8, tail, wb>), grid, block, lds, stream, g.a, \
+                       g.a_scale, g.wq, g.sq, g.c, g.M, g.K, g.N, share, g.bias);                \
     return hipGetLastError();                                                                    \
   }
-#define W4A8_STREAM_FQ_GO(nt, kpw, w, silu, tail)                                                \
+#define W4A8_STREAM_FQ_GO(nt, kpw, w, silu, tail, wb)                                           \
   {                                                                                              \
-    W4A8_STREAM_ATTR((gemm_stream_fq<nt, kpw, w, silu, tail>))                                   \
-    hipLaunchKernelGGL((gemm_stream_fq<nt, kpw, w, silu, tail>), grid, dim3(kFqWaves * 64), lds, \
-                       stream, g.a, g.wq, g.sq, g.c, g.M, g.K, g.N, share, (int)lda);            \
+    W4A8_STREAM_ATTR((gemm_stream_fq<nt, kpw, w, silu, tail, wb>))                             \
+    hipLaunchKernelGGL((gemm_stream_fq<nt, kpw, w, silu, tail, wb>), grid,                     \
+                       dim3(kFqWaves * 64), lds, stream, g.a, g.wq, g.sq, g.c, g.M, g.K, g.N,    \
+                       share, (int)lda, g.bias);                                                 \
     return hipGetLastError();                                                                    \
+  }
+#define W4A8_STREAM_TAIL(go, nt, kpw, w, x, wb)                                                  \
+  {                                                                                              \
+    if (g.K % kKAlign) go(nt, kpw, w, x, true, wb)                                               \
+    go(nt, kpw, w, x, false, wb)                                                                 \
   }
 #define W4A8_STREAM_LAUNCH(nt, kpw, w)                                                           \
   if (idx++ == variant) {                                                                        \
-    const bool tail = g.K % kKAlign != 0;                                                        \
     if constexpr (w >= 4 && w <= kFqWaves - 4 && nt * kpw <= 24) {                               \
-      if (fused && silu && tail) W4A8_STREAM_FQ_GO(nt, kpw, w, true, true)                       \
-      if (fused && silu) W4A8_STREAM_FQ_GO(nt, kpw, w, true, false)                              \
-      if (fused && tail) W4A8_STREAM_FQ_GO(nt, kpw, w, false, true)                              \
-      if (fused) W4A8_STREAM_FQ_GO(nt, kpw, w, false, false)                                     \
+      if (fused && silu) W4A8_STREAM_TAIL(W4A8_STREAM_FQ_GO, nt, kpw, w, true, false)            \
+      if (fused && g.bias) W4A8_STREAM_TAIL(W4A8_STREAM_FQ_GO, nt, kpw, w, false, true)          \
+      if (fused) W4A8_STREAM_TAIL(W4A8_STREAM_FQ_GO, nt, kpw, w, false, false)                   \
     }                                                                                            \
     if (fused) return hipErrorInvalidValue;                                                      \
-    if (g.M <= 8 && tail) W4A8_STREAM_GO(nt, kpw, w, true, true)                                 \
-    if (g.M <= 8) W4A8_STREAM_GO(nt, kpw, w, true, false)                                        \
-    if (tail) W4A8_STREAM_GO(nt, kpw, w, false, true)                                            \
-    W4A8_STREAM_GO(nt, kpw, w, false, false)                                                     \
+    if (g.M <= 8 && g.bias) W4A8_STREAM_TAIL(W4A8_STREAM_GO, nt, kpw, w, true, true)             \
+    if (g.M <= 8) W4A8_STREAM_TAIL(W4A8_STREAM_GO, nt, kpw, w, true, false)                      \
+    if (g.bias) W4A8_STREAM_TAIL(W4A8_STREAM_GO, nt, kpw, w, false, true)                        \
+    W4A8_STREAM_TAIL(W4A8_STREAM_GO, nt, kpw, w, false, false)                                   \
   }
   W4A8_STREAM_TABLE(W4A8_STREAM_LAUNCH)
 #undef W4A8_STREAM_LAUNCH
 #undef W4A8_STREAM_GO
 #undef W4A8_STREAM_FQ_GO
+#undef W4A8_STREAM_TAIL
 #undef W4A8_STREAM_ATTR
   return hipErrorInvalidValue;
 }

@@ -135,7 +135,7 @@ __device__ __forceinline__ void tile_body(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
     const uint32_t* __restrict__ Sq, uint16_t* __restrict__ C, int M, int N, int K, int KTp,
     int KTe, int KG, int NTILES, int grid_m, int grid_n, int ldc, int vec_out,
-    float* __restrict__ P, int splits) {
+    float* __restrict__ P, int splits, const uint16_t* __restrict__ bias) {
   using S = TileShape<WM, WN, NW>;
   static_assert(NS >= 2 && NS <= 16 && (NS - 1) * (S::OPS + 1) < 64, "pipeline depth");
   constexpr int RING = ring_slots(NS);
@@ -525,12 +525,14 @@ __device__ __forceinline__ void tile_body(
     tsc[i] = reinterpret_cast<const float*>(tscale)[(wm * WM + i) * 16 + (lane & 15)];
 
   // Epilogue. A lane holds 4 consecutive columns of one token per MFMA tile, so direct stores
-  // touch 16 rows per instruction (measured: ~7.5 us per 256 x 256 tile on MI355X). A full tile
-  // is therefore staged through the freed pipeline stages, row-major with a 16-byte row pad, and
-  // written out as 16-byte row-contiguous stores; edge tiles store directly.
+  // touch 16 rows per instruction (measured: ~7.5 us per 256 x 256 tile on MI355X). A tile is
+  // therefore staged through the freed pipeline stages, row-major with a 16-byte row pad, and
+  // written out as 16-byte row-contiguous stores (with 16-byte stores N is whole chunks, so a
+  // chunk of an edge tile is all in or all out), where a bias is added too; outputs that take no
+  // 16-byte stores are stored directly.
   constexpr int OROW = S::BN * 2 + 16;
   constexpr bool kStaged = S::BM * OROW <= NS * S::STAGE;
-  if (kStaged && vec_out == 2 && m0 + S::BM <= M && nt_base * kNTile + S::BN <= N) {
+  if (kStaged && vec_out == 2) {
     bare_barrier();                              // every wave is done with the stages
 #pragma unroll
     for (int i = 0; i < WM; ++i) {
@@ -556,10 +558,17 @@ __device__ __forceinline__ void tile_body(
     __syncthreads();
     constexpr int CH = S::BN * 2 / 16;           // 16-byte chunks per row
     uint16_t* const crow = C + (size_t)m0 * ldc + nt_base * kNTile;
+    const bool full = m0 + S::BM <= M && nt_base * kNTile + S::BN <= N;
     for (int idx = tid; idx < S::BM * CH; idx += NW * 64) {
       const int r = idx / CH, c = idx - r * CH;
-      *reinterpret_cast<v4i*>(crow + (size_t)r * ldc + c * 8) =
-          *reinterpret_cast<const v4i*>(lds + r * OROW + c * 16);
+      if (!full && (m0 + r >= M || nt_base * kNTile + c * 8 >= N)) continue;
+      v4i y = *reinterpret_cast<const v4i*>(lds + r * OROW + c * 16);
+      if (bias) {
+        const v4i b = *reinterpret_cast<const v4i*>(bias + nt_base * kNTile + c * 8);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) y[d] = (int)add_bias2((uint32_t)y[d], (uint32_t)b[d]);
+      }
+      *reinterpret_cast<v4i*>(crow + (size_t)r * ldc + c * 8) = y;
     }
     return;
   }
@@ -571,7 +580,7 @@ __device__ __forceinline__ void tile_body(
 #pragma unroll
     for (int j = 0; j < WN; ++j) {
       const int n = (nt_base + wn * WN + j) * kNTile + 4 * (lane >> 4);
-      store_out4(C, ldc, m, n, N, acc[i][j], tsc[i], vec);
+      store_out4(C, ldc, m, n, N, acc[i][j], tsc[i], vec, bias);
     }
   }
 }
@@ -585,19 +594,20 @@ template <int WM, int WN, int NS, int NW, bool AH, bool AT>
 __global__ __launch_bounds__(NW * 64) void gemm_tile(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
     const uint32_t* __restrict__ Sq, uint16_t* __restrict__ C, int M, int N, int K, int KTp,
-    int KTe, int KG, int NTILES, int grid_m, int grid_n, int ldc, int vec_out) {
+    int KTe, int KG, int NTILES, int grid_m, int grid_n, int ldc, int vec_out,
+    const uint16_t* __restrict__ bias) {
   tile_body<WM, WN, NS, NW, AH, AT, false>(A, As, Wq, Sq, C, M, N, K, KTp, KTe, KG, NTILES, grid_m,
-                                       grid_n, ldc, vec_out, nullptr, 1);
+                                       grid_n, ldc, vec_out, nullptr, 1, bias);
 }
 
 template <int WM, int WN, int NS, int NW, bool AH, bool AT>
 __global__ __launch_bounds__(NW * 64) void gemm_tile_pre(
     const uint8_t* __restrict__ A, const float* __restrict__ As, const uint8_t* __restrict__ Wq,
     const uint32_t* __restrict__ Sq, int M, int K, int KTp, int NTILES, int grid_m, int grid_n,
-    int N, int ldc, int vec_out, uint16_t* __restrict__ C) {
+    int N, int ldc, int vec_out, uint16_t* __restrict__ C, const uint16_t* __restrict__ bias) {
   tile_body<WM, WN, NS, NW, AH, AT, false>(A, As, Wq, Sq, C, M, N, K, KTp, ceil_div(K, kKTile),
                                        KTp / kKGroup, NTILES, grid_m, grid_n, ldc, vec_out,
-                                       nullptr, 1);
+                                       nullptr, 1, bias);
 }
 
 // The K-split form of the 4-wave band tiles (WM <= 2): the preloaded argument order of
@@ -608,7 +618,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_tile_split(
     const uint32_t* __restrict__ Sq, int M, int K, int KTp, int NTILES, int grid_m, int grid_n,
     int N, int splits, float* __restrict__ P) {
   tile_body<WM, WN, NS, NW, AH, AT, true>(A, As, Wq, Sq, nullptr, M, N, K, KTp, ceil_div(K, kKTile),
-                                      KTp / kKGroup, NTILES, grid_m, grid_n, N, 0, P, splits);
+                                      KTp / kKGroup, NTILES, grid_m, grid_n, N, 0, P, splits,
+                                      nullptr);
 }
 
 
@@ -653,10 +664,12 @@ hipError_t launch_tile_body(const GemmArgs& g, int variant, bool a_tiled, hipStr
 
 // Adds the `splits` fp32 partial sums P[s][M][N] of a split-K tile launch in split order, scales
 // by the per-token scale and stores bf16: one thread per 4 consecutive columns of one token.
+template <bool BIAS>
 __global__ __launch_bounds__(256) void split_reduce(const float* __restrict__ P,
                                                     const float* __restrict__ As,
                                                     uint16_t* __restrict__ C, int M, int N,
-                                                    int ldc, int splits, int vec_out) {
+                                                    int ldc, int splits, int vec_out,
+                                                    const uint16_t* __restrict__ bias) {
   const int n4 = N >> 2;
   const long idx = (long)blockIdx.x * 256 + threadIdx.x;
   if (idx >= (long)M * n4) return;
@@ -664,15 +677,20 @@ __global__ __launch_bounds__(256) void split_reduce(const float* __restrict__ P,
   const size_t plane = (size_t)M * N, at = (size_t)m * N + n;
   v4f v = *reinterpret_cast<const v4f*>(P + at);
   for (int s = 1; s < splits; ++s) v += *reinterpret_cast<const v4f*>(P + s * plane + at);
-  store_out4(C, ldc, m, n, N, v, As[m], vec_out != 0);
+  store_out4(C, ldc, m, n, N, v, As[m], vec_out != 0, BIAS ? bias : nullptr);
 }
 
 hipError_t launch_split_reduce(const float* partial, const GemmArgs& g, int splits,
                                hipStream_t stream) {
   const long threads = (long)g.M * (g.N / 4);
-  hipLaunchKernelGGL(split_reduce, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream,
-                     partial, g.a_scale, g.c, g.M, g.N, g.ldc, splits,
-                     (g.ldc % 4 == 0 && ((uintptr_t)g.c % 8) == 0) ? 1 : 0);
+  const dim3 grid((unsigned)((threads + 255) / 256));
+  const int vec_out = g.ldc % 4 == 0 && ((uintptr_t)g.c % 8) == 0 ? 1 : 0;
+  if (g.bias)
+    hipLaunchKernelGGL(split_reduce<true>, grid, dim3(256), 0, stream, partial, g.a_scale, g.c, g.M,
+                       g.N, g.ldc, splits, vec_out, g.bias);
+  else
+    hipLaunchKernelGGL(split_reduce<false>, grid, dim3(256), 0, stream, partial, g.a_scale, g.c,
+                       g.M, g.N, g.ldc, splits, vec_out, g.bias);
   return hipGetLastError();
 }
 
@@ -715,11 +733,11 @@ hipError_t launch_tile_body(const GemmArgs& g, int variant, bool a_tiled, hipStr
     } else if constexpr (nw == 8 || wm > 2) {                                                    \
       hipLaunchKernelGGL((gemm_tile<wm, wn, ns, nw, ah, at>), grid, block, 0, stream, g.a,       \
                          g.a_scale, g.wq, g.sq, g.c, g.M, g.N, g.K, KTp, KTe, KG, NTILES, grid_m, \
-                         grid_n, g.ldc, vec_out);                                                \
+                         grid_n, g.ldc, vec_out, g.bias);                                        \
     } else {                                                                                     \
       hipLaunchKernelGGL((gemm_tile_pre<wm, wn, ns, nw, ah, at>), grid, block, 0, stream, g.a,   \
                          g.a_scale, g.wq, g.sq, g.M, g.K, KTp, NTILES, grid_m, grid_n, g.N,      \
-                         g.ldc, vec_out, g.c);                                                   \
+                         g.ldc, vec_out, g.c, g.bias);                                           \
     }                                                                                            \
     return hipGetLastError();                                                                    \
   }

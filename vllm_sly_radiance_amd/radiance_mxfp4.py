@@ -237,9 +237,13 @@ def _mxfp4_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Ten
     M <= 2 (M <= 4 where the plan leaves its quantizing waves little work) one launch quantizes
     beside the streaming GEMM, else two launches; the bits are the same either way. N and K come
     from weight_ref's shape (see module docstring)."""
+    N, K = weight_ref.shape[0], weight_ref.shape[1]
+    return _linear_body(x, weight, weight_scale, N, K, None)
+
+
+def _linear_body(x, weight, weight_scale, N, K, bias):
     STATS["calls"] += 1
     _diag.report_stats(STATS)
-    N, K = weight_ref.shape[0], weight_ref.shape[1]
     if x.dim() != 2 or x.shape[1] != K:
         raise RuntimeError(f"[radiance.mxfp4] x {tuple(x.shape)} does not match K={K}")
     if x.dtype != torch.bfloat16 or x.stride(1) != 1:
@@ -251,7 +255,8 @@ def _mxfp4_linear(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Ten
     q = torch.empty((M, K), dtype=torch.float8_e4m3fn, device=x.device)
     s = torch.empty((M,), dtype=torch.float32, device=x.device)
     _native.linear(x.data_ptr(), x.stride(0), q.data_ptr(), s.data_ptr(), weight.data_ptr(),
-                   weight_scale.data_ptr(), out.data_ptr(), M, N, K, _stream())
+                   weight_scale.data_ptr(), out.data_ptr(), M, N, K, _stream(),
+                   0 if bias is None else bias.data_ptr())
     if _diag.enabled():
         # the one-launch form keeps q in LDS: the check quantizes again (the same bits)
         _diag.after_call(STATS, lambda: quant_per_token(x), None, weight, weight_scale, out, N, K,
@@ -266,6 +271,28 @@ def _mxfp4_linear_fake(x, weight, weight_scale, weight_ref):
 mxfp4_linear = torch.library.custom_op("radiance::mxfp4_linear", _mxfp4_linear, mutates_args=())
 mxfp4_linear.register_fake(_mxfp4_linear_fake)
 call_linear = inference_op(mxfp4_linear, _mxfp4_linear, _mxfp4_linear_fake)
+
+
+def _mxfp4_linear_bias(x: torch.Tensor, weight: torch.Tensor, weight_scale: torch.Tensor,
+                       weight_ref: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
+    """mxfp4_linear(...) + bias in the GEMM's epilogue: the bf16 outputs plus the bf16 bias [N],
+    rounded again, the same bits as the elementwise add. What the epilogue does not take (a bias off
+    16 bytes or strided, diagnostics on) is added afterwards."""
+    N, K = weight_ref.shape[0], weight_ref.shape[1]
+    if bias.dtype != torch.bfloat16 or tuple(bias.shape) != (N,) or bias.stride(0) != 1 \
+            or bias.data_ptr() % 16 or x.shape[0] == 0 or _diag.enabled():
+        return _mxfp4_linear(x, weight, weight_scale, weight_ref) + bias
+    return _linear_body(x, weight, weight_scale, N, K, bias)
+
+
+def _mxfp4_linear_bias_fake(x, weight, weight_scale, weight_ref, bias):
+    return torch.empty((x.shape[0], weight_ref.shape[0]), device=x.device, dtype=torch.bfloat16)
+
+
+mxfp4_linear_bias = torch.library.custom_op("radiance::mxfp4_linear_bias", _mxfp4_linear_bias,
+                                            mutates_args=())
+mxfp4_linear_bias.register_fake(_mxfp4_linear_bias_fake)
+call_linear_bias = inference_op(mxfp4_linear_bias, _mxfp4_linear_bias, _mxfp4_linear_bias_fake)
 
 
 def _mxfp4_linear_pq(x_fp8: torch.Tensor, x_scale: torch.Tensor, weight: torch.Tensor,
@@ -355,6 +382,14 @@ silu_mul_mxfp4_linear = torch.library.custom_op(
 silu_mul_mxfp4_linear.register_fake(_silu_mul_mxfp4_linear_fake)
 call_silu_mul_linear = inference_op(silu_mul_mxfp4_linear, _silu_mul_mxfp4_linear,
                                     _silu_mul_mxfp4_linear_fake)
+
+
+def _fuses_bias(bias, N: int, x: torch.Tensor) -> bool:
+    """Whether the linear's epilogue may add this bias: a bf16 [N] one, outside compilation (an
+    elementwise add is the compiler's to fuse) and where no gradient can be asked for."""
+    return bias is not None and bias.dtype == torch.bfloat16 and bias.dim() == 1 \
+        and bias.shape[0] == N and bias.device == x.device and not torch.compiler.is_compiling() \
+        and not (torch.is_grad_enabled() and (bias.requires_grad or x.requires_grad))
 
 
 # --------------------------------------------------------------------------------------------
@@ -471,9 +506,12 @@ def _make_kernel_class():
                     x_fp8, x_scale, layer.weight, layer.weight_scale, layer.radiance_wref)
             else:
                 lead = x.shape[:-1]
-                y = call_linear(
-                    x.reshape(-1, x.shape[-1]), layer.weight, layer.weight_scale,
-                    layer.radiance_wref)
+                args = (x.reshape(-1, x.shape[-1]), layer.weight, layer.weight_scale,
+                        layer.radiance_wref)
+                if _fuses_bias(bias, layer.radiance_wref.shape[0], x):
+                    y, bias = call_linear_bias(*args, bias), None
+                else:
+                    y = call_linear(*args)
                 y = y.reshape(*lead, y.shape[-1])
             if bias is not None:
                 y = y + bias
