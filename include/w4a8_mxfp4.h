@@ -107,12 +107,11 @@ int w4a8_gemm(const void* a, const float* a_scale, const void* wq, const void* s
 
 /* The plan w4a8_gemm would use: kernel (W4A8_KERNEL_*), variant index and K split. Counterpart of
  * the reference's band/split policy (sly/mxfp4/radiance_mxfp4_fp8.hip:1252-1343, :1390-1500) and
- * its Python replica band_map (sly/mxfp4/band_map.py:31-95). For a macro-tile plan whose
- * workgroups fill a CU each, w4a8_gemm may run the variant on the leading columns that fill whole
- * rounds of workgroups and a 128 x 128 tile variant on the rest (two launches on the stream); the
- * returned triple names the first. For 64 < M <= 1024 the triple names the plan's tile by its
- * throughput table, and w4a8_gemm runs the macro tile that its time-per-slab table prices lowest
- * (the same bits: a macro tile's shape does not change an output's accumulation order). A tile plan with split_k > 1 (the decode band's K split) is
+ * its Python replica band_map (sly/mxfp4/band_map.py:31-95). For M > 64 the triple names the
+ * plan's tile by its throughput table; w4a8_gemm runs the macro tile that its time-per-slab table
+ * prices lowest, or one tile on the leading columns that fill whole rounds of workgroups and
+ * another on the rest (two launches on the stream), with the same bits: a macro tile's shape does
+ * not change an output's accumulation order. A tile plan with split_k > 1 (the decode band's K split) is
  * two launches under w4a8_gemm_planned too: the partial launch and the reducing launch. */
 int w4a8_plan(int M, int N, int K, int* kernel, int* variant, int* split_k);
 

@@ -58,8 +58,6 @@ Scratch g_scratch[kMaxDevices];
 constexpr size_t kUnbounded = ~(size_t)0;
 // The automatic plan splits K across workgroups only in the decode band, M <= kMaxSplitM.
 constexpr int kMaxSplitM = 64;
-// Above the decode band and up to here the automatic path takes mid_tile_auto's tile.
-constexpr int kMidMaxM = 1024;
 const Scratch kPlanAnySplit{nullptr, kUnbounded, nullptr, kUnbounded, "unbounded scratch"};
 
 int current_device() {
@@ -212,8 +210,7 @@ int mid_tile(int M, int N, int cus) {
   return pick;
 }
 
-// What the automatic path runs for 64 < M <= 1024: the tile with the least measured time per 128-k
-// slab, by the rounds of one tile per CU that the shape takes (1, 2 or 3; more in proportion to 3).
+// What the automatic path runs for M > 64: the tile with the least measured time per 128-k slab, by the rounds of one tile per CU that the shape takes (1, 2 or 3; more in proportion to 3).
 // ns per slab on MI355X, medians over 8 decoder shapes (N 3584 .. 28672, K 3584 .. 9472) at M = 65,
 // 80, 96, 128, 160, 192, 200, 224, 256, 320, 384, 448, 512, 640, 768, 900 and 1024, weights
 // rotating through 400 MB, after 4 us of launch, first fill and epilogue. At these M a slab is
@@ -244,18 +241,73 @@ constexpr TileSlab kMidSlabs[] = {
     {4, 8, 8, 3, {1133, 2599, 3900}},   // 256 x 256
 };
 
-int mid_tile_auto(int M, int N, int cus) {
-  double best = 0;
-  int pick = -1;
-  for (const TileSlab& s : kMidSlabs) {
-    const int v = find_tile(s.wm, s.wn, s.nw, s.ns);
-    if (v < 0) continue;
-    const TileCfg c = tile_variant(v);
-    const long rounds = ceil_div((long)ceil_div(M, c.bm) * ceil_div(N, c.bn), (long)cus);
-    const double cost = rounds <= 3 ? s.t[rounds - 1] : s.t[2] * (rounds / 3.0);
-    if (pick < 0 || cost < best) best = cost, pick = v;
+constexpr int kMidSlabCount = sizeof(kMidSlabs) / sizeof(kMidSlabs[0]);
+
+// ns per slab of an M x N region on a tile, and the tile with the least.
+double slab_ns(const TileSlab& s, const TileCfg& c, int M, int N, int cus) {
+  const long rounds = ceil_div((long)ceil_div(M, c.bm) * ceil_div(N, c.bn), (long)cus);
+  return rounds <= 3 ? s.t[rounds - 1] : s.t[2] * (rounds / 3.0);
+}
+
+struct SlabPick {
+  int i;
+  double ns;
+};
+SlabPick least_slab(const int (&variant)[kMidSlabCount], int M, int N, int cus) {
+  SlabPick p{-1, 0};
+  for (int i = 0; i < kMidSlabCount; ++i) {
+    const double ns = slab_ns(kMidSlabs[i], tile_variant(variant[i]), M, N, cus);
+    if (p.i < 0 || ns < p.ns) p = {i, ns};
   }
-  return pick;
+  return p;
+}
+
+// Above the decode band: one tile for all N columns, or one for the leading columns that fill whole
+// rounds of one workgroup per CU and another for the rest, in a launch of its own. A shape whose
+// last round is nearly empty pays a whole round for it (M = 1111 N = 17408 on 256 x 128 tiles: 680
+// tiles, 2.66 rounds), and every tile has other round boundaries; the table prices both launches.
+// Each launch also costs kLaunchNs (start, first fill, epilogue), and a split must save kMinGain
+// of the whole. Measured on MI355X against the picks it replaces (one throughput per tile, only
+// tiles of more than half of a CU's LDS split, only to 128 x 128), weights rotating, us: N = 17408
+// K = 5120 M = 600 / 900 / 1111 / 1400 / 4096 63.2 / 79.3 / 99.6 / 115.8 / 272.4 -> 60.2 / 73.6 /
+// 89.3 / 107.1 / 266.4; N = 28672 K = 4096 M = 600 / 1111 / 1792 81.4 / 129.8 / 182.7 -> 71.2 /
+// 116.3 / 165.4; N = 3584 K = 9472 M = 1111 53.0 -> 40.1; over 62 points of 7 shapes at M = 600 ..
+// 4096 4 % less, and nowhere more than the run-to-run spread (5 %).
+constexpr double kLaunchNs = 4000, kMinGain = 0.03;
+constexpr int kMainTileArea = 128 * 160;
+
+struct ColumnPlan {
+  int n_main, variant, tail;           // tail -1: the one launch covers N
+};
+
+ColumnPlan column_plan(int M, int N, int K, int cus) {
+  struct Variants {
+    int v[kMidSlabCount];
+    Variants() {
+      for (int i = 0; i < kMidSlabCount; ++i)
+        v[i] = find_tile(kMidSlabs[i].wm, kMidSlabs[i].wn, kMidSlabs[i].nw, kMidSlabs[i].ns);
+    }
+  };
+  static const Variants variants;
+  const auto& var = variants.v;
+  const double slabs = ceil_div(K, kKTile);
+  const SlabPick one = least_slab(var, M, N, cus);
+  ColumnPlan best{N, var[one.i], -1};
+  double cost = (kLaunchNs + slabs * one.ns) * (1 - kMinGain);
+  for (int i = 0; i < kMidSlabCount; ++i) {
+    const TileCfg c = tile_variant(var[i]);
+    if (c.bm * c.bn < kMainTileArea) continue;
+    const int mb = ceil_div(M, c.bm), nb = ceil_div(N, c.bn);
+    const int rounds = (int)((long)mb * nb / cus);           // whole rounds that fit, and one less
+    for (int r = rounds; r > 0 && r >= rounds - 1; --r) {
+      const int n = (int)((long)r * cus / mb) * c.bn;
+      if (n <= 0 || n >= N) continue;
+      const SlabPick rest = least_slab(var, M, N - n, cus);
+      const double t = 2 * kLaunchNs + slabs * (slab_ns(kMidSlabs[i], c, M, n, cus) + rest.ns);
+      if (t < cost) cost = t, best = {n, var[i], var[rest.i]};
+    }
+  }
+  return best;
 }
 
 // Prefill candidates (M > 1024), each with its measured throughput per CU (TFLOP/s) over one or
@@ -419,7 +471,7 @@ int plan_tile(int M, int N, int dev) {
     if (tiles(64, 96) <= cus) return find_tile(1, 3, 8, 5);
     return find_tile(2, 4, 4, 4);
   }
-  if (M <= kMidMaxM) return mid_tile(M, N, cus);
+  if (M <= 1024) return mid_tile(M, N, cus);
   return big_tile(M, N, dev);
 }
 
@@ -571,22 +623,15 @@ int gemm_run(const void* a, const float* as, const void* wq, const void* sq, voi
       plan_impl(M, N, K, dev, sc, &kernel, &variant, &split_k);
     }
     if ((kernel == W4A8_KERNEL_TILE || kernel == W4A8_KERNEL_TILE_AT) && M > kMaxSplitM &&
-        M <= kMidMaxM && split_k <= 1) {
-      const int v = mid_tile_auto(M, N, device_info(dev).cus);
-      if (v >= 0) variant = v;
-    }
-    int tail = -1;
-    const int n_main = (kernel == W4A8_KERNEL_TILE || kernel == W4A8_KERNEL_TILE_AT) &&
-                               tile_fits(M, N, K)
-                           ? tile_split(M, N, variant, dev, &tail)
-                           : 0;
-    if (n_main > 0 && n_main < N && n_main % kNTile == 0) {
+        split_k <= 1 && tile_fits(M, N, K)) {
+      const ColumnPlan p = column_plan(M, N, K, device_info(dev).cus);
       const hipStream_t st = (hipStream_t)stream;
-      if (int e = tile_columns(a, as, wq, sq, c, M, N, K, 0, n_main, variant, a_tiled, who, st,
+      if (int e = tile_columns(a, as, wq, sq, c, M, N, K, 0, p.n_main, p.variant, a_tiled, who, st,
                                bias))
         return e;
-      return tile_columns(a, as, wq, sq, c, M, N, K, n_main, N - n_main, tail, a_tiled, who, st,
-                          bias);
+      if (p.tail < 0) return W4A8_OK;
+      return tile_columns(a, as, wq, sq, c, M, N, K, p.n_main, N - p.n_main, p.tail, a_tiled, who,
+                          st, bias);
     }
   }
   return gemm_dispatch(a, as, wq, sq, c, M, N, K, kernel, variant, split_k, sc, who, stream, bias);
