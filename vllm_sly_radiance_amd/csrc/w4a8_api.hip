@@ -989,7 +989,7 @@ W4A8_API int w4a8_silu_mul_quant(const void* gate_up, void* q, float* scale, int
   const size_t part_bytes = sc.partial_bytes;
   return hip_status(launch_silu_mul_quant(gate_up, (uint8_t*)q, scale, nullptr, M, N, part,
                                           part_bytes, q_layout == W4A8_Q_TILED,
-                                          (hipStream_t)stream),
+                                          device_info(current_device()).cus, (hipStream_t)stream),
                     "w4a8_silu_mul_quant");
 }
 
@@ -1036,7 +1036,8 @@ W4A8_API int w4a8_silu_mul(const void* gate_up, void* out, int M, int N, void* s
   if (!aligned(gate_up, 16) || !aligned(out, 16))
     return fail(W4A8_EINVAL, "w4a8_silu_mul: gate_up and out need 16-byte alignment");
   return hip_status(launch_silu_mul_quant(gate_up, nullptr, nullptr, out, M, N, nullptr, 0,
-                                          false, (hipStream_t)stream),
+                                          false, device_info(current_device()).cus,
+                                          (hipStream_t)stream),
                     "w4a8_silu_mul");
 }
 

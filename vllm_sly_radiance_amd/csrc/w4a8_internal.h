@@ -159,7 +159,7 @@ hipError_t launch_add_rms_quant(const void* y, const void* res, const void* w, u
 // `out` set (bf16 [M, N]) it writes the bf16 stage instead of quantizing, one workgroup per row.
 size_t producer_split_bytes(int M, int N);
 hipError_t launch_silu_mul_quant(const void* gate_up, uint8_t* q, float* scale, void* out, int M,
-                                 int N, void* part, size_t part_bytes, bool tiled,
+                                 int N, void* part, size_t part_bytes, bool tiled, int cus,
                                  hipStream_t stream);
 // diagnostic: the producers' fp32 silu of 8 * groups bf16 inputs (16-byte aligned), unrounded
 hipError_t launch_silu_probe(const void* x, float* y, int groups, hipStream_t stream);

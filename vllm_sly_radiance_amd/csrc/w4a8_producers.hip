@@ -201,6 +201,112 @@ __global__ __launch_bounds__(T) void silu_mul_quant(const uint4* __restrict__ gu
   quant_tail<G, T>(nb, nv, q, scale, row, tiled);
 }
 
+// ---- silu_mul at many rows: bf16(silu(gate)) from a table --------------------------------------
+// silu of a bf16 gate, rounded to bf16, is a function of 16 bits. A row per workgroup computes it
+// anew for every element (~27 vector operations, and a division each in a wave that holds a gate
+// past 44 in magnitude: 50 us for 4096 rows of 8704 on MI355X, of which the 178 MB take ~30).
+// Here a workgroup first tabulates it for every gate of magnitude 2^-13 .. 2^7 with the same steps
+// (5120 values, one 8-value group per thread, as fp32 in 26 KiB of LDS) and then takes rows
+// blockIdx, blockIdx + gridDim, ..., one lookup per element; groups that hold a gate outside the
+// table (zeros, infinities and NaNs among them) are computed as before, so the bits are the same.
+// The next row's loads go out before the current row's reduction. 640 threads: one table group
+// each, and 2 x 640 or 3 x 640 groups cover rows of 8704, 9472 and 14336 with few idle lanes (1024
+// threads measured 42.8 us at 4096 x 8704 where 640 take 37.6). Measured on MI355X, one launch, gates
+// of standard deviation 2 / 20 (us, before -> now): N = 8704 M = 200 7.0 -> 5.8 / 8.0 -> 5.5,
+// M = 1111 16.6 -> 13.1 / 20.0 -> 12.8, M = 4096 43.8 -> 37.6 / 50.5 -> 36.8 (4.8 TB/s);
+// N = 14336 M = 1111 25.6 -> 20.2 / 31.0 -> 20.1; N = 17408 M = 1111 30.0 -> 24.2 / 36.1 -> 23.4.
+constexpr int kLutT = 640;
+constexpr uint32_t kLutLo = (127 - 13) << 7;     // bf16 magnitude bits of 2^-13
+constexpr int kLutN = 20 << 7;                   // to below 2^7
+constexpr int kLutSign = 4096;                   // entry of -x: that of x + 4096
+
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint4 silu_mul_lut(const float* tab, const uint4 gv, const uint4 uv) {
+  const uint32_t g[4] = {gv.x, gv.y, gv.z, gv.w}, u[4] = {uv.x, uv.y, uv.z, uv.w};
+  const u16x2 lo = {(unsigned short)kLutLo, (unsigned short)kLutLo};
+  u16x2 e[4], top;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    e[i] = __builtin_bit_cast(u16x2, g[i] & 0x7FFF7FFFu) - lo;     // below 2^-13: wraps past kLutN
+    top = i ? __builtin_elementwise_max(top, e[i]) : e[i];
+  }
+  if (__builtin_expect(max((uint32_t)top[0], (uint32_t)top[1]) >= (uint32_t)kLutN, 0))
+    return silu_mul_group(gv, uv);
+  float p[8];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t d = __builtin_bit_cast(uint32_t, e[i]);
+    p[2 * i] = tab[(d & 0xFFFFu) + ((g[i] >> 3) & 0x1000u)] * __uint_as_float(u[i] << 16);
+    p[2 * i + 1] = tab[(d >> 16) + ((g[i] >> 19) & 0x1000u)] * __uint_as_float(u[i] & 0xFFFF0000u);
+  }
+  return pack8_hw(p);
+}
+
+template <int G>
+__global__ __launch_bounds__(kLutT, G <= 2 ? 5 : 3) void silu_mul_quant_lut(const uint4* __restrict__ gu,
+                                                            uint8_t* __restrict__ q,
+                                                            float* __restrict__ scale, int M, int N,
+                                                            int tiled) {
+  __shared__ float tab[kLutSign + kLutN];
+  __shared__ uint32_t red[2][kLutT / 64];
+  const int tid = threadIdx.x, nv = N >> 3;
+  uint4 gv[G], uv[G];
+  int row = blockIdx.x;
+  {
+    const uint4* gate = gu + (size_t)row * 2 * nv;
+    load_groups<G, kLutT>(gate, nv, gv, uv, gate + nv);
+  }
+  static_assert(2 * kLutN == 8 * kLutT, "a table group per thread");
+  {
+    const int neg = tid >= kLutN / 8, e = 8 * (tid - neg * (kLutN / 8));
+    float x[8], y[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      x[j] = __uint_as_float((kLutLo + e + j + (neg ? 0x8000u : 0u)) << 16);
+    silu8(x, y);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) tab[neg * kLutSign + e + j] = bf16_round_hw(y[j]);
+  }
+  __syncthreads();
+  for (int it = 0; row < M; row += gridDim.x, ++it) {
+    uint4 nb[G];
+    uint32_t am = 0;
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+      if (tid + i * kLutT < nv) {
+        nb[i] = silu_mul_lut(tab, gv[i], uv[i]);
+        am = max(am, abs_bits_max8(nb[i]));
+      }
+    }
+    const int next = row + gridDim.x;
+    if (next < M) {                              // uniform: the next row, behind this one's tail
+      const uint4* gate = gu + (size_t)next * 2 * nv;
+      load_groups<G, kLutT>(gate, nv, gv, uv, gate + nv);
+    }
+    // the row maximum; two buffers, so one barrier per row keeps a row's reads from the next writes
+    am = wave_max(am);
+    if ((tid & 63) == 0) red[it & 1][tid >> 6] = am;
+    __builtin_amdgcn_s_waitcnt(0xC07F);          // lgkmcnt(0); the next row's loads stay in flight
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    uint32_t m = red[it & 1][0];
+#pragma unroll
+    for (int w = 1; w < kLutT / 64; ++w) m = max(m, red[it & 1][w]);
+    const float sc = row_scale(m);
+    const float rcp = 1.0f / sc;
+    if (tid == 0) scale[row] = sc;
+#pragma unroll
+    for (int i = 0; i < G; ++i) {
+      const int g = tid + i * kLutT;
+      if (g < nv)
+        *reinterpret_cast<uint2*>(q + q_offset(row, g, nv, tiled)) =
+            quant8_any_scale(nb[i], sc, rcp);
+    }
+  }
+}
+
 // One 8-element group of the per-head gated RMSNorm from its loaded x, z and weight groups. All 16
 // lanes of a head call it together. It runs on every lane of a wave that holds part of the row: a
 // group past the row holds zeros (the result is finite and never stored), and with no branch per
@@ -356,8 +462,18 @@ hipError_t launch_add_rms_quant(const void* y, const void* res, const void* w, u
 // Rows of work per CU: with fewer rows than half the CUs, each row takes a 1024-thread workgroup.
 constexpr int kWideRowsMax = 128;
 
+// Where silu_mul looks its silu up: above the rows that take 1024-thread workgroups, and where the
+// elements saved pay for the tables. Gates of standard deviation 2, us computed / looked up: N = 8704
+// M = 130 6.6 / 5.9; N = 6144 M = 400 / 768 / 1111 6.9 / 7.6, 8.9 / 9.0, 11.6 / 11.3; N = 4352
+// M = 1111 / 2048 9.2 / 9.4, 14.2 / 13.6 (deviation 20, where a computed group divides: 7.7 / 5.4,
+// 7.8 / 7.3, 10.3 / 8.8, 14.2 / 11.0, 11.1 / 9.0, 17.1 / 13.2).
+bool silu_lookup(int M, int N) {
+  if (M <= kWideRowsMax) return false;
+  return N > 8192 || (N > 5120 && M >= 1024) || (N > 4096 && M >= 2048);
+}
+
 hipError_t launch_silu_mul_quant(const void* gate_up, uint8_t* q, float* scale, void* out, int M,
-                                 int N, void* part, size_t part_bytes, bool tiled,
+                                 int N, void* part, size_t part_bytes, bool tiled, int cus,
                                  hipStream_t stream) {
   if (M == 0) return hipSuccess;
   if (!out && split_rows(M, N, part, part_bytes)) {
@@ -367,6 +483,19 @@ hipError_t launch_silu_mul_quant(const void* gate_up, uint8_t* q, float* scale, 
     hipLaunchKernelGGL(silu_mul_quant_split<true>, dim3(S, M), dim3(64), 0, stream,
                        (const uint4*)gate_up, q, scale, (uint32_t*)part, N, S, (int)tiled);
     return hipGetLastError();
+  }
+  if (!out && silu_lookup(M, N)) {
+    // two workgroups per CU, or one where a thread's three or four groups need the registers
+    const int per_cu = N <= 2 * 8 * kLutT ? 2 : 1;
+    const dim3 grid(M < per_cu * cus ? M : per_cu * cus);
+#define W4A8_SMQ_LUT(C)                                                                         \
+  if (N <= C * 8 * kLutT) {                                                                     \
+    hipLaunchKernelGGL(silu_mul_quant_lut<C>, grid, dim3(kLutT), 0, stream,                     \
+                       (const uint4*)gate_up, q, scale, M, N, (int)tiled);                      \
+    return hipGetLastError();                                                                   \
+  }
+    W4A8_SMQ_LUT(1) W4A8_SMQ_LUT(2) W4A8_SMQ_LUT(3) W4A8_SMQ_LUT(4)
+#undef W4A8_SMQ_LUT
   }
   const bool wide = M <= kWideRowsMax;
   const int T = wide ? 1024 : kThreads;
