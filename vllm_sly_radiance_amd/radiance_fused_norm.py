@@ -70,10 +70,6 @@ GDN_MAX_N = 10240
 GDN_HEAD = 128
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
-
-
 def _need_bf16(op: str, **tensors: torch.Tensor) -> None:
     bad = {k: t.dtype for k, t in tensors.items() if t.dtype != torch.bfloat16}
     if bad:
@@ -127,7 +123,7 @@ def _add_rms_quant(y: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor
     if M:
         y, residual, weight = y.contiguous(), residual.contiguous(), weight.contiguous()
         _native.add_rms_quant(y.data_ptr(), residual.data_ptr(), weight.data_ptr(), q.data_ptr(),
-                              s.data_ptr(), r.data_ptr(), M, K, float(eps), _stream(),
+                              s.data_ptr(), r.data_ptr(), M, K, float(eps), _rmx._stream(),
                               _layout(q, M, K, tiled))
     return q, s, r
 
@@ -154,7 +150,7 @@ def _silu_mul_quant(gate_up: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     q, s = _qs(M, N, gate_up.device, tiled)
     if M:
         gate_up = gate_up.contiguous()
-        _native.silu_mul_quant(gate_up.data_ptr(), q.data_ptr(), s.data_ptr(), M, N, _stream(),
+        _native.silu_mul_quant(gate_up.data_ptr(), q.data_ptr(), s.data_ptr(), M, N, _rmx._stream(),
                                _layout(q, M, N, tiled))
     return q, s
 
@@ -184,7 +180,7 @@ def _gdn_norm_quant(x: torch.Tensor, z: torch.Tensor, weight: torch.Tensor,
         x, weight = x.contiguous(), weight.contiguous()
         z, zs = _row_runs(z, N)
         _native.gdn_norm_quant(x.data_ptr(), z.data_ptr(), zs, weight.data_ptr(), q.data_ptr(),
-                               s.data_ptr(), M, N, float(eps), _stream(), _layout(q, M, N, tiled))
+                               s.data_ptr(), M, N, float(eps), _rmx._stream(), _layout(q, M, N, tiled))
     return q, s
 
 
