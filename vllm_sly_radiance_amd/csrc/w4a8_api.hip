@@ -311,8 +311,8 @@ ColumnPlan column_plan(int M, int N, int K, int cus) {
 }
 
 // Prefill candidates (M > 1024), each with its measured throughput per CU (TFLOP/s) over one or
-// more full rounds of one workgroup per CU, and that of the 128 x 128 tiles the automatic path
-// gives the columns of a ragged last round (tile_split). Measured on MI355X, every candidate on
+// more full rounds of one workgroup per CU, and that of 128 x 128 tiles on the columns of a ragged
+// last round (tile_split). Measured on MI355X, every candidate on
 // the four Qwen3.8-27B linear shapes at M = 1280, 1536, 2048, 2560, 3072 and 4096 with warm
 // clocks (medians).
 constexpr TileRate kBigTiles[] = {
@@ -331,8 +331,8 @@ double round_cost(int M, int N, const TileCfg& c, float rate, int cus) {
   return per * ((double)c.bm * c.bn) / rate;
 }
 
-// M > 1024: the candidate with the least predicted time as the automatic path would run it (its
-// ragged last round split off to 128 x 128 tiles where tile_split does so). Rounds are what
+// M > 1024: the tile the plan names, the candidate with the least predicted time (a ragged last
+// round split off to 128 x 128 tiles where tile_split does so; column_plan prices what runs). Rounds are what
 // matter here: at M = 1280 .. 3072 the best tile is the one whose tiles fill whole rounds (qkv
 // M = 1280: 256 x 256 in one round of 200 tiles, 56.9 us, against 80 us for 256 x 160 in 320
 // tiles; o_proj and down M = 2560, 3072: 256 x 256 at 66.5-92.9 us against 90.6-122 us). Over the
@@ -477,8 +477,8 @@ int plan_tile(int M, int N, int dev) {
 
 // A tile variant whose workgroup fills a CU's LDS runs in rounds of one workgroup per CU. When the
 // last round would run at under half occupancy (gate/up at M = 4096 on 256 x 256 tiles: 1088
-// tiles = 4.25 rounds), the automatic path gives the variant the columns [0, n_main) that fill
-// whole rounds (16384 of 17408) and the rest to 128 x 128 tiles, which fill one more, shorter
+// tiles = 4.25 rounds), big_tile prices the variant on the columns [0, n_main) that fill
+// whole rounds (16384 of 17408) and the rest on 128 x 128 tiles, which fill one more, shorter
 // round. Returns n_main, or 0 for no split.
 int tile_split(int M, int N, int variant, int dev, int* tail_variant) {
   const TileCfg c = tile_variant(variant);
