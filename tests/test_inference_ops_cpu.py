@@ -1,5 +1,9 @@
 """The direct registration of each custom op (radiance::<name>_inference): the public op's schema and
 body, taken only where no gradient can be asked for and nothing is compiled."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -53,3 +57,54 @@ def test_fake_tensors_and_tracing_see_the_op():
     assert any("probe_fake_inference" in str(n.target) for n in graph.graph.nodes)
     with torch.inference_mode():
         assert torch.equal(call(torch.ones(2)), torch.full((2,), 2.0))
+
+
+def test_the_modules_can_be_loaded_again():
+    """importlib.reload and a fresh import register every op again: the newest body runs, also for
+    calls through the earlier module, and reloading one module leaves the other's ops alone."""
+    code = """
+import gc, importlib, sys, torch
+def check(R, F):
+    gc.collect()
+    x = torch.empty(3, 64, dtype=torch.bfloat16, device="meta")
+    w, ws, ref = (torch.empty(s, dtype=torch.uint8, device="meta") for s in ((32, 32), (32, 2), (32, 64, 0)))
+    assert R.call_linear(x, w, ws, ref).shape == torch.ops.radiance.mxfp4_linear(x, w, ws, ref).shape == (3, 32)
+    assert R.call_linear_bias(x, w, ws, ref, x[0, :32]).shape == (3, 32)
+    q, s = F.call_silu_mul_quant(x)
+    assert q.shape == (3, 32) and s.shape == (3,)
+from vllm_sly_radiance_amd import radiance_mxfp4 as R, radiance_fused_norm as F
+check(R, F)
+for module in (R, R, F, R):
+    importlib.reload(module)
+    check(R, F)
+old = R, F
+for name in [n for n in sys.modules if n.startswith("vllm_sly_radiance_amd")]:
+    del sys.modules[name]
+import vllm_sly_radiance_amd.radiance_mxfp4 as R, vllm_sly_radiance_amd.radiance_fused_norm as F
+assert R is not old[0]
+check(R, F)
+check(*old)
+del old
+check(R, F)
+
+def probe(factor):
+    def body(x: torch.Tensor) -> torch.Tensor:
+        return x * factor
+    op = torch.library.custom_op("radiance::probe_again", body, mutates_args=())
+    return R.inference_op(op, body, torch.empty_like)
+first, second = probe(2.0), probe(3.0)
+with torch.no_grad():
+    assert first(torch.ones(1)).item() == second(torch.ones(1)).item() == 3.0
+def wider(x: torch.Tensor, factor: float) -> torch.Tensor:
+    return x * factor
+op = torch.library.custom_op("radiance::probe_again", wider, mutates_args=())
+assert R.inference_op(op, wider, lambda x, factor: torch.empty_like(x))(torch.ones(1), 5.0).item() == 5.0
+first, second = probe(2.0), probe(3.0)
+grad = torch.ones(1, requires_grad=True)
+assert first(grad).item() == second(grad).item() == 3.0
+print("ok")
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    run = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True,
+                         timeout=120)
+    assert run.returncode == 0 and run.stdout.strip() == "ok", run.stderr

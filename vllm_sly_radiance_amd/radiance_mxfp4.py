@@ -21,6 +21,7 @@ from __future__ import annotations
 
 import os
 import sys
+import warnings
 from collections import OrderedDict
 
 import torch
@@ -215,7 +216,26 @@ def gemm(x_fp8: torch.Tensor, x_scale: torch.Tensor, weight: torch.Tensor,
 # --------------------------------------------------------------------------------------------
 # Custom ops: the whole path is one opaque node (sly/mxfp4/radiance_mxfp4.py:644-652)
 # --------------------------------------------------------------------------------------------
-_fragment = torch.library.Library("radiance", "FRAGMENT")
+def _register_direct(ns, name, schema, body, fake):
+    """Registers body and fake as ns::name. Defining a name twice in a process raises, so where this
+    module is loaded again (importlib.reload, a fresh import) they replace the earlier ones, as
+    torch.library.custom_op does for the public op. The operator holds the Library objects: an op is
+    removed with the one that defined it, and calls made through the earlier module would follow.
+    None where an earlier load defined the name with another schema."""
+    space = getattr(torch.ops, ns)
+    again = hasattr(space, name)
+    if again and str(getattr(space, name).default._schema) != f"{ns}::{schema}":
+        return None
+    lib = torch.library.Library(ns, "FRAGMENT")
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore")          # the dispatcher says that a kernel is replaced
+        if not again:
+            lib.define(schema)
+        lib.impl(name, body, "CompositeExplicitAutograd", allow_override=again)
+        torch.library.register_fake(f"{ns}::{name}", fake, lib=lib, allow_override=again)
+    direct = getattr(space, name).default
+    direct.__dict__.setdefault("_radiance_libraries", []).append(lib)
+    return direct
 
 
 def inference_op(op, body, fake):
@@ -226,16 +246,14 @@ def inference_op(op, body, fake):
     on the GPU). Returns a callable that takes the second form where no gradient can be asked for
     and nothing is being compiled, and `op` (whose backward raises) otherwise."""
     ns, name = op._qualname.split("::")
-    schema = str(op._opoverload._schema)
-    _fragment.define(schema.replace(f"{ns}::{name}(", f"{name}_inference(", 1))
-    _fragment.impl(f"{name}_inference", body, "CompositeExplicitAutograd")
-    torch.library.register_fake(f"{ns}::{name}_inference", fake)
-    public, direct = op._opoverload, getattr(torch.ops.radiance, f"{name}_inference").default
+    direct = _register_direct(ns, f"{name}_inference", str(op._opoverload._schema).replace(
+        f"{ns}::{name}(", f"{name}_inference(", 1), body, fake)
+    space = getattr(torch.ops, ns)               # the public op by name: a reload replaces it
 
     def call(*args):
-        if torch.compiler.is_compiling() or (torch.is_grad_enabled() and any(
+        if direct is None or torch.compiler.is_compiling() or (torch.is_grad_enabled() and any(
                 a.requires_grad for a in args if isinstance(a, torch.Tensor))):
-            return public(*args)
+            return getattr(space, name)(*args)
         return direct(*args)
     return call
 
