@@ -1,5 +1,6 @@
 """The direct registration of each custom op (radiance::<name>_inference): the public op's schema and
-body, taken only where no gradient can be asked for and nothing is compiled."""
+body, taken only where no gradient can be asked for and nothing compiles, traces or watches ops by
+name."""
 import os
 import subprocess
 import sys
@@ -53,10 +54,45 @@ def test_fake_tensors_and_tracing_see_the_op():
     with FakeTensorMode():
         assert call(torch.empty(4, 5)).shape == (4, 5)
     assert not calls
-    graph = make_fx(call, tracing_mode="fake")(torch.ones(2))
-    assert any("probe_fake_inference" in str(n.target) for n in graph.graph.nodes)
+    for how in (dict(tracing_mode="real"), dict(tracing_mode="fake"), dict(pre_dispatch=True)):
+        graph = make_fx(call, **how)(torch.ones(2))
+        assert [str(n.target) for n in graph.graph.nodes][1:-1] == ["radiance.probe_fake.default"], how
+    assert "radiance::probe_fake(" in str(torch.jit.trace(call, torch.ones(2), check_trace=False).graph)
     with torch.inference_mode():
         assert torch.equal(call(torch.ones(2)), torch.full((2,), 2.0))
+
+
+def test_modes_and_subclasses_see_the_public_op():
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    call, _ = _probe("probe_modes")
+    seen = []
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    class Sub(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    x = torch.ones(2)
+    for mode in (Dispatch, Function):
+        with mode():
+            call(x)
+    call(x.as_subclass(Sub))
+    assert [s.removesuffix(".default") for s in seen if "probe" in s] == ["radiance.probe_modes"] * 3
+    with torch.device("cpu"):                    # a default device is a function mode, and not one
+        assert not R._watched()                  # that looks at ops
+    assert not R._watched()
 
 
 def test_the_modules_can_be_loaded_again():

@@ -25,6 +25,7 @@ import warnings
 from collections import OrderedDict
 
 import torch
+from torch.utils._device import DeviceContext
 
 from . import _native
 from . import diagnostics as _diag
@@ -238,21 +239,42 @@ def _register_direct(ns, name, schema, body, fake):
     return direct
 
 
+_compiling, _jit_tracing = torch.compiler.is_compiling, torch._C._is_tracing
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+
+
+def _watched() -> bool:
+    """Whether something sees ops by name here: a compiler, a tracer (make_fx before or after
+    autograd, torch.jit.trace), a dispatch mode, or a function mode other than a default device."""
+    return _compiling() or _dispatch_modes() > 0 or _jit_tracing() or (
+        _function_modes() > 0 and not all(isinstance(torch._C._get_function_stack_at(i), DeviceContext)
+                                          for i in range(_function_modes())))
+
+
+def _asks_gradient(args) -> bool:
+    for a in args:
+        if isinstance(a, torch.Tensor) and a.requires_grad:
+            return True
+    return False
+
+
 def inference_op(op, body, fake):
     """A second registration of the custom op `op`, radiance::<name>_inference: the same schema and
     body straight on the dispatcher, without custom_op's Python autograd and alias-checking layers.
     Those take ~9.5 of the ~14 us a custom_op call costs before its body, more than the GPU time of a
     small linear (one token through N = 10240 K = 5120, called from Python: 21 us a call, 6 of them
     on the GPU). Returns a callable that takes the second form where no gradient can be asked for
-    and nothing is being compiled, and `op` (whose backward raises) otherwise."""
+    and nothing watches ops by name, and `op` (whose backward raises, and whose name a graph or a
+    mode then sees) otherwise. A body returns new tensors: the layers left out are what refuses one
+    that returns its input."""
     ns, name = op._qualname.split("::")
     direct = _register_direct(ns, f"{name}_inference", str(op._opoverload._schema).replace(
         f"{ns}::{name}(", f"{name}_inference(", 1), body, fake)
     space = getattr(torch.ops, ns)               # the public op by name: a reload replaces it
 
     def call(*args):
-        if direct is None or torch.compiler.is_compiling() or (torch.is_grad_enabled() and any(
-                a.requires_grad for a in args if isinstance(a, torch.Tensor))):
+        if direct is None or _watched() or type(args[0]) is not torch.Tensor \
+                or (torch.is_grad_enabled() and _asks_gradient(args)):
             return getattr(space, name)(*args)
         return direct(*args)
     return call
