@@ -95,6 +95,36 @@ def test_modes_and_subclasses_see_the_public_op():
     assert not R._watched()
 
 
+def test_a_bias_that_something_differentiates_or_maps_is_added_outside(monkeypatch):
+    """Forward-mode tangents of the bias, vmap over it and traced graphs need its add as an op of its
+    own; a plain call takes the epilogue."""
+    from types import SimpleNamespace
+
+    import torch.autograd.forward_ad as fw
+    from torch.fx.experimental.proxy_tensor import make_fx
+    x, y = torch.ones(2, 32, dtype=torch.bfloat16), torch.full((2, 4), 3.0, dtype=torch.bfloat16)
+    layer = SimpleNamespace(weight=None, weight_scale=None, radiance_wref=torch.empty(4, 32, 0))
+    fused = []
+    monkeypatch.setattr(R, "call_linear", lambda *args: y.clone())
+    monkeypatch.setattr(R, "call_linear_bias", lambda *args: fused.append(1) or y + args[-1])
+    bias = torch.arange(4.0).bfloat16()
+
+    def apply(b):
+        return R.kernel_class()().apply(layer, x, b)
+
+    assert torch.equal(apply(bias), y + bias) and len(fused) == 1
+    with fw.dual_level():
+        out = fw.unpack_dual(apply(fw.make_dual(bias, torch.full_like(bias, 2.0))))
+    assert torch.equal(out.primal, y + bias) and (out.tangent == 2).all()
+    out, tangent = torch.func.jvp(apply, (bias,), (torch.full_like(bias, 2.0),))
+    assert torch.equal(out, y + bias) and (tangent == 2).all()
+    biases = torch.stack([bias, bias + 1])
+    assert torch.equal(torch.func.vmap(apply)(biases), y + biases[:, None])
+    names = [str(n.target) for n in make_fx(apply)(bias).graph.nodes]
+    assert "aten.add.Tensor" in names
+    assert len(fused) == 1
+
+
 def test_the_modules_can_be_loaded_again():
     """importlib.reload and a fresh import register every op again: the newest body runs, also for
     calls through the earlier module, and reloading one module leaves the other's ops alone."""

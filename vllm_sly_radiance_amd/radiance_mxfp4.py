@@ -25,6 +25,7 @@ import warnings
 from collections import OrderedDict
 
 import torch
+from torch.autograd import forward_ad
 from torch.utils._device import DeviceContext
 
 from . import _native
@@ -434,10 +435,13 @@ call_silu_mul_linear = inference_op(silu_mul_mxfp4_linear, _silu_mul_mxfp4_linea
 
 
 def _fuses_bias(bias, N: int, x: torch.Tensor) -> bool:
-    """Whether the linear's epilogue may add this bias: a bf16 [N] one, outside compilation (an
-    elementwise add is the compiler's to fuse) and where no gradient can be asked for."""
+    """Whether the linear's epilogue may add this bias: a bf16 [N] one, where no gradient or tangent
+    of it can be asked for, no transform (vmap, functionalize) maps it and nothing watches ops by name
+    (an elementwise add is a compiler's or tracer's to see)."""
     return bias is not None and bias.dtype == torch.bfloat16 and bias.dim() == 1 \
-        and bias.shape[0] == N and bias.device == x.device and not torch.compiler.is_compiling() \
+        and bias.shape[0] == N and bias.device == x.device and not _watched() \
+        and torch._C._functorch.peek_interpreter_stack() is None \
+        and forward_ad._current_level < 0 \
         and not (torch.is_grad_enabled() and (bias.requires_grad or x.requires_grad))
 
 
