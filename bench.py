@@ -749,7 +749,9 @@ def bench_sweep(n_layers):
                                                     for k, v in per_shape.items()},
                             tflops=round(flop / (ms * 1e-3) / 1e12, 1),
                             gbs=round(nbytes / (ms * 1e-3) / 1e9, 1),
-                            plans={name: list(_native.plan(M, N, K)) for name, N, K in LAYER_M1}))
+                            plans={name: list(_native.plan(M, N, K)) for name, N, K in LAYER_M1},
+                            plan_columns={name: list(_native.plan_columns(M, N, K))
+                                          for name, N, K in LAYER_M1}))
         print(f"[bench] sweep M={M}: {ms:.3f} ms per forward of {n_layers} layers "
               f"({forward[-1]['per_shape_us_per_layer']} us per layer)", file=sys.stderr,
               flush=True)
@@ -759,7 +761,7 @@ def bench_sweep(n_layers):
     # kernel with the fragments covering M (its first variant that serves the shape; a forced
     # plan, kept to show why the plan takes the tiles there), timed on row-major q and, as
     # ring_at_us, on the same codes fragment-tiled (contiguous 1 KiB activation loads instead of
-    # 16 token rows x 64 bytes); the tile family is the macro tile the plan takes at M, or at
+    # 16 token rows x 64 bytes); the tile family is the macro tiles the plan takes at M, or at
     # M = 17 below that, with the plan's K split (tile_split; tile_unsplit_us beside it). From 17
     # to 64 tokens band_us is the fastest band-kernel variant (weight waves and activation waves)
     # that serves the shape unsplit; where the plan takes the band kernel, plan_us is the plan.
@@ -797,8 +799,9 @@ def bench_sweep(n_layers):
             else:
                 tile_v, tile_sp = (v, sp) if k == _native.KERNEL_TILE else \
                     _native.plan(max(M, 17), N, K)[1:]
-            row["tile_us"] = round(_timed_graph(
-                lambda: run(_native.KERNEL_TILE, tile_v, tile_sp), 5) * 1e3 / per, 2)
+            # above 64 tokens the automatic path: the plan may give the last columns another tile
+            tile = (_native.KERNEL_TILE, tile_v, tile_sp) if M <= 64 else (_native.KERNEL_AUTO, -1, 0)
+            row["tile_us"] = round(_timed_graph(lambda: run(*tile), 5) * 1e3 / per, 2)
             if 16 < M <= 64:
                 # every band variant that serves the shape unsplit; the fastest is reported
                 band = []

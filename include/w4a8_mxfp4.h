@@ -107,13 +107,18 @@ int w4a8_gemm(const void* a, const float* a_scale, const void* wq, const void* s
 
 /* The plan w4a8_gemm would use: kernel (W4A8_KERNEL_*), variant index and K split. Counterpart of
  * the reference's band/split policy (sly/mxfp4/radiance_mxfp4_fp8.hip:1252-1343, :1390-1500) and
- * its Python replica band_map (sly/mxfp4/band_map.py:31-95). For M > 64 the triple names the
- * plan's tile by its throughput table; w4a8_gemm runs the macro tile that its time-per-slab table
- * prices lowest, or one tile on the leading columns that fill whole rounds of workgroups and
- * another on the rest (two launches on the stream), with the same bits: a macro tile's shape does
- * not change an output's accumulation order. A tile plan with split_k > 1 (the decode band's K split) is
- * two launches under w4a8_gemm_planned too: the partial launch and the reducing launch. */
+ * its Python replica band_map (sly/mxfp4/band_map.py:31-95). For M > 64 the triple names the macro
+ * tile of the first launch, which covers all N or the leading columns that fill whole rounds of
+ * workgroups; w4a8_plan_columns names the rest. Under w4a8_gemm_planned the triple covers all N in
+ * one launch, with the same bits: a macro tile's shape does not change an output's accumulation
+ * order. A tile plan with split_k > 1 (the decode band's K split) is two launches there too: the
+ * partial launch and the reducing launch. */
 int w4a8_plan(int M, int N, int K, int* kernel, int* variant, int* split_k);
+
+/* The columns of w4a8_plan's launches: the first covers [0, n_main), and where n_main < N a second
+ * one, on the stream behind it, covers [n_main, N) with macro-tile variant tail_variant (-1: one
+ * launch, n_main == N). No counterpart in the reference. */
+int w4a8_plan_columns(int M, int N, int K, int* n_main, int* tail_variant);
 
 /* The GEMM on fragment-tiled activations (W4A8_Q_TILED, as the producers write them; K % 128 == 0):
  * the macro-tile kernel with the plan w4a8_gemm would take for a macro tile at this (M, N) (the

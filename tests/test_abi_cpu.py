@@ -171,21 +171,18 @@ def test_one_launch_linear_where_it_pays(lib):
     (32, 17408, 5120, (32, 96)), (32, 65536, 5120, (32, 128)),
     (33, 5120, 6144, (32, 64)), (64, 17408, 5120, (64, 96)), (64, 5120, 8704, (32, 64)),
     (64, 10240, 5120, (64, 64)), (64, 65536, 5120, (64, 128)),
-    # 64 < M <= 1024: the candidate with the least predicted time (tiles per CU x area / rate);
-    # these are the measured-fastest variants at those points on MI355X
-    (65, 10240, 5120, (32, 128)), (128, 10240, 5120, (64, 128)), (384, 10240, 5120, (128, 128)),
-    (512, 10240, 5120, (256, 128)), (1024, 10240, 5120, (256, 160)),
-    (128, 5120, 6144, (32, 128)), (384, 5120, 8704, (64, 128)), (768, 5120, 8704, (128, 128)),
-    (1024, 5120, 8704, (256, 128)),
-    (96, 17408, 5120, (128, 128)), (192, 17408, 5120, (64, 128)), (256, 17408, 5120, (256, 128)),
-    (512, 17408, 5120, (256, 160)), (768, 17408, 5120, (256, 256)), (1024, 17408, 5120, (256, 160)),
-    # M > 1024: the candidate (256 x 128, 256 x 160, 256 x 256, 128 x 256) whose rounds of
-    # one-per-CU workgroups, with a ragged last round split off where the path splits it, take
-    # the least predicted time
+    # above 64 tokens: the tile of the first launch that the automatic path runs, with the least
+    # measured time per slab (test_plan_columns: what covers the columns it leaves)
+    (65, 10240, 5120, (32, 128)), (128, 10240, 5120, (64, 96)), (384, 10240, 5120, (128, 128)),
+    (512, 10240, 5120, (128, 160)), (1024, 10240, 5120, (256, 160)),
+    (128, 5120, 6144, (32, 96)), (384, 5120, 8704, (64, 128)), (768, 5120, 8704, (128, 128)),
+    (1024, 5120, 8704, (128, 160)),
+    (96, 17408, 5120, (64, 160)), (192, 17408, 5120, (128, 160)), (256, 17408, 5120, (128, 160)),
+    (512, 17408, 5120, (256, 160)), (768, 17408, 5120, (256, 256)), (1024, 17408, 5120, (256, 256)),
     (1280, 10240, 5120, (256, 256)), (1280, 5120, 6144, (256, 128)),
     (2048, 5120, 6144, (256, 160)), (2560, 5120, 8704, (256, 256)),
     (2048, 17408, 5120, (256, 256)), (4096, 17408, 5120, (256, 256)),
-    (4096, 10240, 5120, (256, 160)), (4096, 5120, 8704, (256, 256))])
+    (4096, 10240, 5120, (256, 256)), (4096, 5120, 8704, (256, 256))])
 def test_plan_tile_shapes(lib, M, N, K, tile):
     k, v, s = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     assert lib.w4a8_plan(M, N, K, ctypes.byref(k), ctypes.byref(v), ctypes.byref(s)) == 0
@@ -193,12 +190,55 @@ def test_plan_tile_shapes(lib, M, N, K, tile):
     assert _native.variants(2)[v.value][2:] == tile
 
 
+@pytest.mark.parametrize("M,N,K,n_main,tail", [
+    # two launches: the columns that fill whole rounds of 256 x 256 tiles, the rest on smaller ones
+    (1111, 17408, 5120, 13056, (128, 160)), (4096, 17408, 5120, 16384, (128, 128)),
+    (4096, 5120, 8704, 4096, (128, 128)), (1024, 17408, 5120, 16384, (64, 64)),
+    (2048, 17408, 5120, 16384, (64, 128)), (4096, 10240, 5120, 8192, (256, 128)),
+    # one: whole rounds, a K so short that a second launch costs more than it saves, and every plan
+    # up to 64 tokens (streaming, skinny, band, split and unsplit tiles)
+    (768, 17408, 5120, None, None), (4096, 4608, 256, None, None), (1111, 1288, 512, None, None),
+    (1, 17408, 5120, None, None), (8, 33, 640, None, None), (40, 17408, 5120, None, None),
+    (24, 5120, 8704, None, None), (64, 65536, 5120, None, None)])
+def test_plan_columns(lib, M, N, K, n_main, tail):
+    """The second launch of a macro-tile plan: its tile and the columns it starts at."""
+    if n_main is None:
+        assert _native.plan_columns(M, N, K) == (N, -1)
+        return
+    n, v = _native.plan_columns(M, N, K)
+    assert (n, _native.variants(2)[v][2:]) == (n_main, tail)
+
+
+def test_plan_columns_are_whole_tiles_of_the_first_launch(lib):
+    """Over a sweep of shapes: w4a8_plan names a tile that serves the shape, and where it leaves
+    columns to a second launch they start at a whole tile of it."""
+    split = 0
+    for M in (65, 100, 200, 513, 600, 777, 1024, 1111, 1500, 2048, 3001, 4096):
+        for N in (1000, 1024, 3584, 5120, 10240, 17408, 28672, 32768):
+            for K in (256, 640, 4096, 9472):
+                k, v, s = _native.plan(M, N, K)
+                n, tail = _native.plan_columns(M, N, K)
+                assert (k, s) == (_native.KERNEL_TILE, 1)
+                assert _native.variant_serves(k, v, M, n, K)
+                if tail < 0:
+                    assert n == N
+                    continue
+                split += 1
+                assert 0 < n < N and n % _native.tile_config(v)["bn"] == 0
+                assert _native.variant_serves(k, tail, M, N - n, K)
+    assert split > 50
+    n, v = ctypes.c_int(), ctypes.c_int()
+    assert lib.w4a8_plan_columns(100, 512, 40, ctypes.byref(n), ctypes.byref(v)) == 1
+    assert lib.w4a8_plan_columns(100, 512, 512, None, ctypes.byref(v)) == 1
+
+
 @pytest.mark.parametrize("M,N,K,stages,waves", [
     (17, 5120, 6144, 8, 4), (32, 17408, 5120, 8, 4), (64, 5120, 8704, 8, 4),
     (64, 10240, 5120, 5, 4), (64, 17408, 5120, 5, 8), (96, 5120, 8704, 8, 4),
-    (96, 17408, 5120, 4, 8), (4096, 17408, 5120, 3, 8)])
+    (96, 17408, 5120, 5, 4), (4096, 17408, 5120, 3, 8)])
 def test_plan_pipeline_depth_and_waves(lib, M, N, K, stages, waves):
-    """Narrow tiles run 8 stages deep (latency-bound at these M); large tiles 3-5, in 8 waves."""
+    """Narrow tiles run 8 stages deep (latency-bound at these M); large tiles 3-5, the largest in 8
+    waves."""
     k, v, s = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     assert lib.w4a8_plan(M, N, K, ctypes.byref(k), ctypes.byref(v), ctypes.byref(s)) == 0
     c = _native.tile_config(v.value)

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from oracle import mxfp4_oracle as O
+from vllm_sly_radiance_amd import _native
 from vllm_sly_radiance_amd import diagnostics as D
 from vllm_sly_radiance_amd import synthetic
 
@@ -72,6 +73,15 @@ def test_checkall_reports_ok_then_wrong(diag, capsys):
     nan[0, 0] = float("nan")
     diag.after_call(stats, lambda: (q, s), None, wq, sq, nan, N, K)   # NaN counts as wrong
     assert stats["wrong"] == 2 and stats["checked"] == 4
+
+
+def test_mhist_names_both_tiles_of_a_two_launch_plan(diag, capsys):
+    M, N, K = 1111, 17408, 5120
+    n_main, tail = _native.plan_columns(M, N, K)
+    assert 0 < n_main < N
+    diag.after_call({}, None, None, None, None, torch.empty((M, N), device="meta"), N, K)
+    assert (f"M={M} plan=tile variant={_native.plan(M, N, K)[1]} split_k=1 columns={n_main} "
+            f"rest_variant={tail}\n") in capsys.readouterr().err
 
 
 def test_checkall_skips_other_shapes_large_m_and_capture(diag, capsys, monkeypatch):

@@ -35,6 +35,7 @@ SIGNATURES = {
     "w4a8_gemm_at": (_int, [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _vp]),
     "w4a8_tiled_bytes": (_int, [_int, _int, _psz]),
     "w4a8_plan": (_int, [_int, _int, _int, _pint, _pint, _pint]),
+    "w4a8_plan_columns": (_int, [_int, _int, _int, _pint, _pint]),
     "w4a8_gemm_planned": (_int, [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _int, _int,
                                  _vp]),
     "w4a8_gemm_noalloc": (_int, [_vp, _vp, _vp, _vp, _vp, _int, _int, _int, _int, _int, _int,
@@ -203,6 +204,14 @@ def plan(M: int, N: int, K: int):
     k, v, s = _int(), _int(), _int()
     check(lib().w4a8_plan(M, N, K, _c.byref(k), _c.byref(v), _c.byref(s)))
     return k.value, v.value, s.value
+
+
+def plan_columns(M: int, N: int, K: int):
+    """(n_main, tail variant) of plan()'s launches: the second tile covers columns n_main .. N - 1;
+    (N, -1) for one launch."""
+    n, v = _int(), _int()
+    check(lib().w4a8_plan_columns(M, N, K, _c.byref(n), _c.byref(v)))
+    return n.value, v.value
 
 
 def variants(kernel: int):

@@ -171,55 +171,18 @@ int find_stream(int M, int N, int K, int dev) {
   return best;
 }
 
-// Macro-tile candidates above the decode band, each with its measured throughput per CU
-// (TFLOP/s) with one workgroup on the CU (r1) and with two workgroups' worth of tiles per CU (r2,
-// running together or in two rounds). Measured on MI355X, every variant on the four Qwen3.8-27B
-// linear shapes at M = 65, 96, 128, 192, 256, 384, 512, 768 and 1024 (medians over the cases with
-// that many tiles per CU).
-struct TileRate {
-  int wm, wn, nw, ns;
-  float r1, r2;
-};
-constexpr TileRate kMidTiles[] = {
-    {2, 2, 4, 5, 3.77f, 4.59f},    // 64 x 64
-    {1, 4, 4, 8, 3.79f, 3.74f},    // 32 x 128, 8 stages
-    {2, 4, 4, 4, 5.60f, 6.24f},    // 64 x 128
-    {2, 4, 8, 4, 8.09f, 7.83f},    // 128 x 128, 8 waves
-    {2, 8, 8, 4, 9.77f, 9.51f},    // 128 x 256, 8 waves
-    {4, 4, 8, 3, 11.53f, 9.96f},   // 256 x 128, 8 waves
-    {4, 5, 8, 3, 12.28f, 10.09f},  // 256 x 160, 8 waves
-    {4, 8, 8, 3, 13.65f, 12.41f},  // 256 x 256, 8 waves
-};
-
-// 64 < M <= 1024: the candidate with the least predicted time, tiles per CU x tile area / rate
-// (r2 when the tiles come two per CU). Against the fastest variant measured at each of the 36
-// points above, the pick is 0.5 % slower on average and 5.7 % at worst (gate_up M = 384); the
-// first-fit rule it replaces was up to 33 % slower (qkv M = 384: 35.7 against 23.7 us).
-int mid_tile(int M, int N, int cus) {
-  double best = 0;
-  int pick = -1;
-  for (const TileRate& t : kMidTiles) {
-    const int v = find_tile(t.wm, t.wn, t.nw, t.ns);
-    if (v < 0) continue;
-    const TileCfg c = tile_variant(v);
-    const long per = ceil_div((long)ceil_div(M, c.bm) * ceil_div(N, c.bn), (long)cus);
-    const double area = (double)c.bm * c.bn;
-    const double cost = per == 2 ? 2 * area / t.r2 : per * area / t.r1;
-    if (pick < 0 || cost < best) best = cost, pick = v;
-  }
-  return pick;
-}
-
-// What the automatic path runs for M > 64: the tile with the least measured time per 128-k slab, by the rounds of one tile per CU that the shape takes (1, 2 or 3; more in proportion to 3).
+// The macro tile for M > 64: the one with the least measured time per 128-k slab, by the rounds of
+// one tile per CU that the shape takes (1, 2 or 3; more in proportion to 3).
 // ns per slab on MI355X, medians over 8 decoder shapes (N 3584 .. 28672, K 3584 .. 9472) at M = 65,
 // 80, 96, 128, 160, 192, 200, 224, 256, 320, 384, 448, 512, 640, 768, 900 and 1024, weights
 // rotating through 400 MB, after 4 us of launch, first fill and epilogue. At these M a slab is
-// bound by LDS traffic (a 128 x 128 slab's fragment reads and fills take ~340 ns of LDS time against
-// ~215 ns of MFMA), so tiles whose waves own more columns per token row (a column is 64 bytes of a
-// slab, a token 128) and that read their fragments a slab ahead do best. Against the fastest tile at
-// each of the 136 points the pick is 0.4 % slower on average; against the throughput table above,
-// whose picks the plan names, it is 7 % faster (N = 17408 M = 200: 31.7 -> 27.5 us, N = 10240
-// M = 200 / 512: 21.4 -> 17.4, 32.7 -> 27.9, N = 5120 K = 8704 M = 200: 22.7 -> 18.9).
+// bound by LDS traffic (a 128 x 128 slab moves 64 KiB of fragment reads and 24 KiB of fills
+// through LDS against ~215 ns of MFMA), so tiles whose waves own more columns per token row (a
+// column is 64 bytes of a slab, a token 128) and that read their fragments a slab ahead do best.
+// Against the fastest tile at each of the 136 points the pick is 0.4 % slower on average; a table
+// of one throughput per tile, the rule before, picked 7 % slower ones (N = 17408 M = 200 31.7
+// against 27.5 us, N = 10240 M = 200 / 512 21.4 / 32.7 against 17.4 / 27.9, N = 5120 K = 8704
+// M = 200 22.7 against 18.9).
 struct TileSlab {
   int wm, wn, nw, ns;
   int t[3];
@@ -266,13 +229,14 @@ SlabPick least_slab(const int (&variant)[kMidSlabCount], int M, int N, int cus) 
 // rounds of one workgroup per CU and another for the rest, in a launch of its own. A shape whose
 // last round is nearly empty pays a whole round for it (M = 1111 N = 17408 on 256 x 128 tiles: 680
 // tiles, 2.66 rounds), and every tile has other round boundaries; the table prices both launches.
+// A tile's shape does not change an output's accumulation order, so neither choice changes bits.
 // Each launch also costs kLaunchNs (start, first fill, epilogue), and a split must save kMinGain
-// of the whole. Measured on MI355X against the picks it replaces (one throughput per tile, only
-// tiles of more than half of a CU's LDS split, only to 128 x 128), weights rotating, us: N = 17408
-// K = 5120 M = 600 / 900 / 1111 / 1400 / 4096 63.2 / 79.3 / 99.6 / 115.8 / 272.4 -> 60.2 / 73.6 /
-// 89.3 / 107.1 / 266.4; N = 28672 K = 4096 M = 600 / 1111 / 1792 81.4 / 129.8 / 182.7 -> 71.2 /
-// 116.3 / 165.4; N = 3584 K = 9472 M = 1111 53.0 -> 40.1; over 62 points of 7 shapes at M = 600 ..
-// 4096 4 % less, and nowhere more than the run-to-run spread (5 %).
+// of the whole. Measured on MI355X against one throughput per tile with a split to 128 x 128 where
+// the last round was under half full, weights rotating, us: N = 17408 K = 5120 M = 600 / 900 / 1111
+// / 1400 / 4096 63.2 / 79.3 / 99.6 / 115.8 / 272.4 -> 60.2 / 73.6 / 89.3 / 107.1 / 266.4;
+// N = 28672 K = 4096 M = 600 / 1111 / 1792 81.4 / 129.8 / 182.7 -> 71.2 / 116.3 / 165.4; N = 3584
+// K = 9472 M = 1111 53.0 -> 40.1; over 62 points of 7 shapes at M = 600 .. 4096 4 % less, and
+// nowhere more than the run-to-run spread (5 %).
 constexpr double kLaunchNs = 4000, kMinGain = 0.03;
 constexpr int kMainTileArea = 128 * 160;
 
@@ -310,60 +274,13 @@ ColumnPlan column_plan(int M, int N, int K, int cus) {
   return best;
 }
 
-// Prefill candidates (M > 1024), each with its measured throughput per CU (TFLOP/s) over one or
-// more full rounds of one workgroup per CU, and that of 128 x 128 tiles on the columns of a ragged
-// last round (tile_split). Measured on MI355X, every candidate on
-// the four Qwen3.8-27B linear shapes at M = 1280, 1536, 2048, 2560, 3072 and 4096 with warm
-// clocks (medians).
-constexpr TileRate kBigTiles[] = {
-    {4, 4, 8, 3, 9.75f, 0.f},   // 256 x 128
-    {4, 5, 8, 3, 10.36f, 0.f},  // 256 x 160
-    {4, 8, 8, 3, 12.11f, 0.f},  // 256 x 256
-    {2, 8, 8, 4, 9.14f, 0.f},   // 128 x 256
-};
-constexpr float kSplitTailRate = 8.3f;
-
-int tile_split(int M, int N, int variant, int dev, int* tail_variant);
-
-// Rounds of one-per-CU workgroups for an M x N GEMM on tile c, times area / rate.
-double round_cost(int M, int N, const TileCfg& c, float rate, int cus) {
-  const long per = ceil_div((long)ceil_div(M, c.bm) * ceil_div(N, c.bn), (long)cus);
-  return per * ((double)c.bm * c.bn) / rate;
-}
-
-// M > 1024: the tile the plan names, the candidate with the least predicted time (a ragged last
-// round split off to 128 x 128 tiles where tile_split does so; column_plan prices what runs). Rounds are what
-// matter here: at M = 1280 .. 3072 the best tile is the one whose tiles fill whole rounds (qkv
-// M = 1280: 256 x 256 in one round of 200 tiles, 56.9 us, against 80 us for 256 x 160 in 320
-// tiles; o_proj and down M = 2560, 3072: 256 x 256 at 66.5-92.9 us against 90.6-122 us). Over the
-// 21 measured points whose pick runs as one launch or whose split was timed, the pick is 0.1 %
-// slower than the fastest candidate on average and 1.7 % at worst.
-int big_tile(int M, int N, int dev) {
-  const int cus = device_info(dev).cus;
-  double best = 0;
-  int pick = -1;
-  for (const TileRate& t : kBigTiles) {
-    const int v = find_tile(t.wm, t.wn, t.nw, t.ns);
-    if (v < 0) continue;
-    const TileCfg c = tile_variant(v);
-    double cost = round_cost(M, N, c, t.r1, cus);
-    int tail = -1;
-    const int n_main = tile_split(M, N, v, dev, &tail);
-    if (n_main > 0 && n_main < N && n_main % kNTile == 0)
-      cost = round_cost(M, n_main, c, t.r1, cus) +
-             round_cost(M, N - n_main, tile_variant(tail), kSplitTailRate, cus);
-    if (pick < 0 || cost < best) best = cost, pick = v;
-  }
-  return pick;
-}
-
 // Decode / verify band: M <= 16 takes the streaming family when a variant fits (whole-K
 // workgroups, every weight load in flight at once), else the skinny family, whose workgroup count
 // should cover the 256 CUs several times over (for small N the K dimension is split across
-// workgroups too). Above 16 tokens the macro tiles (plan_tile). The ring kernel is not in the
+// workgroups too). Above 16 tokens the macro tiles (tile_plan). The ring kernel is not in the
 // automatic plan: the 8-stage narrow tiles beat it at every M from 17 to 64 on the four
 // Qwen3.8-27B shapes (it stays available to a forced plan).
-int plan_tile(int M, int N, int dev);
+ColumnPlan tile_plan(int M, int N, int K, int cus);
 
 // Decode band, K split across workgroup rows (the tile kernel writes fp32 partials, a second launch
 // adds them in split order). At these M every workgroup streams the whole M x K activation panel
@@ -395,8 +312,10 @@ int band_split(int M, int N, int K, int cus, const Scratch& sc, int* variant) {
   return kBandSplit;
 }
 
+// cols: the columns of each launch, a second one for an unsplit macro-tile plan only.
 void plan_impl(int M, int N, int K, int dev, const Scratch& sc, int* kernel, int* variant,
-               int* split_k) {
+               int* split_k, ColumnPlan* cols = nullptr) {
+  if (cols) *cols = {N, -1, -1};
   if (M <= 16) {
     const int v = find_stream(M, N, K, dev);
     if (v >= 0) {
@@ -441,11 +360,14 @@ void plan_impl(int M, int N, int K, int dev, const Scratch& sc, int* kernel, int
   }
   *kernel = W4A8_KERNEL_TILE;
   *split_k = band_split(M, N, K, d.cus, sc, variant);
-  if (*split_k == 1) *variant = plan_tile(M, N, dev);
+  if (*split_k > 1) return;
+  const ColumnPlan p = tile_plan(M, N, K, d.cus);
+  *variant = p.variant;
+  if (cols) *cols = p;
 }
 
-// The macro-tile variant for an M x N GEMM: the decode-band rule for M <= 64, the prefill rule
-// below otherwise. Fragment-tiled activations always take this plan.
+// The macro tiles of an unsplit M x N x K GEMM: the decode-band rule for M <= 64, column_plan
+// above. Fragment-tiled activations always take this plan.
 //
 // Decode band (measured on MI355X, every tile variant up to 64 x 96 and every ring variant on the
 // four Qwen3.8-27B linear shapes at M = 17 .. 64): the tiles are latency-bound here, so they run 8
@@ -457,44 +379,22 @@ void plan_impl(int M, int N, int K, int dev, const Scratch& sc, int* kernel, int
 //    workgroups; o_proj 9.6-9.9, down 12.1-13.2 us against 11.4-15.4 on 64-token tiles), else
 //    64 x 64 (qkv, 160 workgroups, 11.8-13.2 us), else 64 x 96 in 8 waves (gate_up, 182
 //    workgroups, 14.7-15.9 us).
-int plan_tile(int M, int N, int dev) {
-  const int cus = device_info(dev).cus;
+int band_tile(int M, int N, int cus) {
   auto tiles = [&](int bm, int bn) { return (long)ceil_div(M, bm) * ceil_div(N, bn); };
   if (M <= 32) {
     int wn = 1;
     while (wn < 4 && tiles(32, 32 * wn) > cus) ++wn;
     return wn < 4 ? find_tile(1, wn, 4, 8) : find_tile(1, 4, 4, 4);
   }
-  if (M <= 64) {
-    if (tiles(32, 64) <= cus) return find_tile(1, 2, 4, 8);
-    if (tiles(64, 64) <= cus) return find_tile(2, 2, 4, 5);
-    if (tiles(64, 96) <= cus) return find_tile(1, 3, 8, 5);
-    return find_tile(2, 4, 4, 4);
-  }
-  if (M <= 1024) return mid_tile(M, N, cus);
-  return big_tile(M, N, dev);
+  if (tiles(32, 64) <= cus) return find_tile(1, 2, 4, 8);
+  if (tiles(64, 64) <= cus) return find_tile(2, 2, 4, 5);
+  if (tiles(64, 96) <= cus) return find_tile(1, 3, 8, 5);
+  return find_tile(2, 4, 4, 4);
 }
 
-// A tile variant whose workgroup fills a CU's LDS runs in rounds of one workgroup per CU. When the
-// last round would run at under half occupancy (gate/up at M = 4096 on 256 x 256 tiles: 1088
-// tiles = 4.25 rounds), big_tile prices the variant on the columns [0, n_main) that fill
-// whole rounds (16384 of 17408) and the rest on 128 x 128 tiles, which fill one more, shorter
-// round. Returns n_main, or 0 for no split.
-int tile_split(int M, int N, int variant, int dev, int* tail_variant) {
-  const TileCfg c = tile_variant(variant);
-  const DeviceInfo d = device_info(dev);
-  if ((size_t)2 * c.lds <= d.lds) return 0;       // two or more workgroups per CU
-  const int mb = ceil_div(M, c.bm), nb = ceil_div(N, c.bn), slots = d.cus;
-  const long total = (long)mb * nb;
-  if (total < slots || total % slots == 0 || 2 * (total % slots) >= slots) return 0;
-  int nbm = nb - 1;
-  while (nbm > 0 && ((long)mb * nbm) % slots) --nbm;
-  // the tail's 128 x 128 tiles: 4 stages when they fit one round (the plan's rule)
-  const long tail_tiles = (long)ceil_div(M, 128) * ceil_div(N - nbm * c.bn, 128);
-  const int tv = find_tile(4, 4, 4, tail_tiles <= slots ? 4 : 3);
-  if (nbm <= 0 || tv < 0) return 0;
-  *tail_variant = tv;
-  return nbm * c.bn;
+ColumnPlan tile_plan(int M, int N, int K, int cus) {
+  if (M > kMaxSplitM) return column_plan(M, N, K, cus);
+  return {N, band_tile(M, N, cus), -1};
 }
 
 // Output columns [n0, n0 + n) of an M x N GEMM on one tile variant: the weights, scales and
@@ -598,7 +498,7 @@ int gemm_dispatch(const void* a, const float* as, const void* wq, const void* sq
 
 // The GEMM on one scratch view: validation, the automatic plan (kernel == W4A8_KERNEL_AUTO) or
 // the forced one, and the launch(es) on `stream`. a_tiled: the activations are fragment-tiled,
-// which the tile kernel alone reads (the automatic plan is then plan_tile's).
+// which the tile kernel alone reads (the automatic plan is then tile_plan's).
 int gemm_run(const void* a, const float* as, const void* wq, const void* sq, void* c, int M, int N,
              int K, int kernel, int variant, int split_k, bool a_tiled, const Scratch& sc,
              const char* who, void* stream, const uint16_t* bias = nullptr) {
@@ -615,23 +515,25 @@ int gemm_run(const void* a, const float* as, const void* wq, const void* sq, voi
   if (int e = check_gemm_ptrs(who, a, as, wq, sq, c)) return e;
   if (kernel == W4A8_KERNEL_AUTO) {
     const int dev = current_device();
+    ColumnPlan cols{N, -1, -1};
     if (a_tiled) {
+      const int cus = device_info(dev).cus;
       kernel = W4A8_KERNEL_TILE_AT;
-      split_k = band_split(M, N, K, device_info(dev).cus, sc, &variant);
-      if (split_k == 1) variant = plan_tile(M, N, dev);
+      split_k = band_split(M, N, K, cus, sc, &variant);
+      if (split_k == 1) {
+        cols = tile_plan(M, N, K, cus);
+        variant = cols.variant;
+      }
     } else {
-      plan_impl(M, N, K, dev, sc, &kernel, &variant, &split_k);
+      plan_impl(M, N, K, dev, sc, &kernel, &variant, &split_k, &cols);
     }
-    if ((kernel == W4A8_KERNEL_TILE || kernel == W4A8_KERNEL_TILE_AT) && M > kMaxSplitM &&
-        split_k <= 1 && tile_fits(M, N, K)) {
-      const ColumnPlan p = column_plan(M, N, K, device_info(dev).cus);
+    if (cols.tail >= 0 && tile_fits(M, N, K)) {
       const hipStream_t st = (hipStream_t)stream;
-      if (int e = tile_columns(a, as, wq, sq, c, M, N, K, 0, p.n_main, p.variant, a_tiled, who, st,
+      if (int e = tile_columns(a, as, wq, sq, c, M, N, K, 0, cols.n_main, variant, a_tiled, who, st,
                                bias))
         return e;
-      if (p.tail < 0) return W4A8_OK;
-      return tile_columns(a, as, wq, sq, c, M, N, K, p.n_main, N - p.n_main, p.tail, a_tiled, who,
-                          st, bias);
+      return tile_columns(a, as, wq, sq, c, M, N, K, cols.n_main, N - cols.n_main, cols.tail,
+                          a_tiled, who, st, bias);
     }
   }
   return gemm_dispatch(a, as, wq, sq, c, M, N, K, kernel, variant, split_k, sc, who, stream, bias);
@@ -701,6 +603,18 @@ W4A8_API int w4a8_plan(int M, int N, int K, int* kernel, int* variant, int* spli
   if (!kernel || !variant || !split_k) return fail(W4A8_EINVAL, "w4a8_plan: null output");
   const int dev = current_device();
   plan_impl(M, N, K, dev, registered_scratch(dev), kernel, variant, split_k);
+  return W4A8_OK;
+}
+
+W4A8_API int w4a8_plan_columns(int M, int N, int K, int* n_main, int* tail_variant) {
+  if (int e = check_gemm_shape("w4a8_plan_columns", M, N, K)) return e;
+  if (!n_main || !tail_variant) return fail(W4A8_EINVAL, "w4a8_plan_columns: null output");
+  const int dev = current_device();
+  int kernel = 0, variant = -1, split_k = 1;
+  ColumnPlan cols{N, -1, -1};
+  plan_impl(M, N, K, dev, registered_scratch(dev), &kernel, &variant, &split_k, &cols);
+  *n_main = cols.n_main;
+  *tail_variant = cols.tail;
   return W4A8_OK;
 }
 

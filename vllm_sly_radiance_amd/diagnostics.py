@@ -183,8 +183,10 @@ def after_call(stats: dict, x_fp8, x_scale, wq, sq, out, N: int, K: int, x=None)
     if MHIST and ("m", N, K, M) not in _seen:
         _seen.add(("m", N, K, M))
         k, v, s = _native.plan(M, N, K) if M else (0, -1, 1)
+        n_main, tail = _native.plan_columns(M, N, K) if M else (N, -1)
+        rest = f" columns={n_main} rest_variant={tail}" if tail >= 0 else ""
         sys.stderr.write(f"[radiance.mxfp4.mhist] N={N} K={K} M={M} "
-                         f"plan={KERNEL_NAMES.get(k, k)} variant={v} split_k={s}\n")
+                         f"plan={KERNEL_NAMES.get(k, k)} variant={v} split_k={s}{rest}\n")
         sys.stderr.flush()
     debug = (DEBUG and not capturing and 0 < M <= 128 and ("d", N, K, M) not in _seen
              and sum(1 for k in _seen if k[0] == "d") < DEBUG_MAX)
