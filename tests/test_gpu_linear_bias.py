@@ -1,8 +1,9 @@
 """The linear with its bias in the GEMM epilogue against the linear followed by the elementwise add, bit
 for bit, on each kernel of the automatic plan: the one-launch linear, the streaming GEMM (two
 widths, K of whole and part k-groups), skinny with and without its K split, band, tiles with staged
-and direct stores, the K-split tiles with their reduction, and the two-launch prefill; N off the
-vector width, and biases the epilogue does not take."""
+and direct stores, the K-split tiles with their reduction, and two tiles side by side in two
+launches; N off the vector width, NaN, infinite and overflowing sums, and biases the epilogue does
+not take. test_bias_epilogue_on_its_route holds each shape to the kernel it is there for."""
 import pytest
 import torch
 
@@ -42,6 +43,62 @@ def test_bias_epilogue_equals_the_add(gpu_lib, M, N, K):
     assert R.STATS["calls"] == before + 1
     x3 = x.reshape(1, M, K)
     assert torch.equal(kern.apply(layer, x3, bias), (y + bias).reshape(1, M, N))
+
+
+def route(M, N, K):
+    """The epilogue that a biased linear of this shape runs through."""
+    kernel, _, split = _native.plan(M, N, K)
+    if kernel == _native.KERNEL_STREAM:
+        return "one launch" if _native.linear_fused(M, N, K, K) else "stream"
+    if kernel in (_native.KERNEL_SKINNY, _native.KERNEL_TILE) and split > 1:
+        return ("skinny" if kernel == _native.KERNEL_SKINNY else "tile") + ", K split"
+    if kernel == _native.KERNEL_TILE:
+        two = ", two launches" if _native.plan_columns(M, N, K)[1] >= 0 else ""
+        return ("tile, staged" if N % 8 == 0 else "tile, direct") + two
+    return {_native.KERNEL_SKINNY: "skinny", _native.KERNEL_BAND: "band"}[kernel]
+
+
+ROUTES = [(1, 5120, 4352, "one launch"), (2, 10240, 1024, "one launch"), (8, 301, 1024, "stream"),
+          (13, 5120, 4352, "stream"), (16, 2070, 640, "skinny"), (16, 1000, 640, "skinny, K split"),
+          (5, 40, 8288, "skinny, K split"), (16, 301, 8288, "skinny, K split"),
+          (40, 10240, 5120, "band"), (33, 8195, 640, "band"),
+          (24, 5120, 8704, "tile, K split"), (200, 1024, 640, "tile, staged"),
+          (200, 1004, 640, "tile, direct"), (77, 1003, 640, "tile, direct"),
+          (1111, 16384, 1024, "tile, staged, two launches"),
+          (513, 13824, 2560, "tile, staged, two launches"),
+          (520, 13852, 2560, "tile, direct, two launches"),
+          (1300, 13827, 1024, "tile, direct, two launches")]
+
+
+@pytest.mark.parametrize("M,N,K,path", ROUTES)
+def test_bias_epilogue_on_its_route(gpu_lib, M, N, K, path):
+    """Token 0 holds a NaN, token 1 zeros, the last token's activations are near bf16's largest so that
+    outputs overflow, and the bias holds NaNs of either sign, infinities and zeros of both signs,
+    the largest bf16 and a subnormal, at the first columns, the last and those of a second launch.
+    Bits of the add, a NaN for a NaN, canonical (its sign is the hardware's choice of operand)."""
+    layer, kern = loaded(N, K), R.kernel_class()()
+    assert route(M, N, K) == path
+    x = bf16_dev(synthetic.activations(M, K, seed=M))
+    x[M - 1] = torch.where(x[M - 1] < 0, -3.0e38, 3.0e38).bfloat16()
+    if M > 1:
+        x[0, K - 1] = float("nan")
+    if M > 2:
+        x[1] = 0
+    bias = 0.1 * torch.randn(N, device="cuda").bfloat16()
+    special = torch.tensor([0x7FC0, -0x40, 0x7F81, 0x7F80, -0x80, 0, -0x8000, 0x7F7F, -0x81, 1],
+                           dtype=torch.int16, device="cuda").view(torch.bfloat16)
+    for at in {0, 7, N - 10, _native.plan_columns(M, N, K)[0] % N}:
+        bias[at:at + 10] = special
+    assert R._fuses_bias(bias, N, x)
+    y = kern.apply(layer, x)
+    out, want = kern.apply(layer, x, bias), y + bias
+    assert torch.isinf(y[M - 1]).any() and not torch.isnan(y[M - 1]).any()
+    nan = torch.isnan(want)
+    assert M == 1 or nan[0].all()
+    assert torch.equal(torch.isnan(out), nan)
+    bits, want_bits = out.view(torch.int16), want.view(torch.int16)
+    assert torch.equal(bits[~nan], want_bits[~nan])
+    assert (bits[nan] & 0x7FFF == 0x7FC0).all()
 
 
 def test_biases_the_epilogue_does_not_take(gpu_lib):
