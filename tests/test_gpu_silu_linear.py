@@ -56,10 +56,12 @@ def same(a, b, what):
     assert bad.size == 0, f"{what}: {len(bad)} outputs differ, first {bad[:3].tolist()}"
 
 
-# the benchmark's down projection (one launch at M <= 2), a 5120-wide square one, and shapes whose
-# plan has no room for quantizing waves (two launches at every M)
-@pytest.mark.parametrize("N,K,one_up_to", [(5120, 8704, 2), (5120, 5120, 2), (2048, 1024, 0),
-                                           (1040, 512, 0)])
+# the benchmark's down projection (one launch at M <= 2), a 5120-wide square one, three whose last
+# k-group is part padding (4352 = 8.5, 3968 = 7.75, 4224 = 8.25 k-groups), and shapes whose plan has
+# no room for quantizing waves (two launches at every M; 9472 = 18.5 k-groups)
+@pytest.mark.parametrize("N,K,one_up_to", [(5120, 8704, 2), (5120, 5120, 2), (5120, 4352, 2),
+                                           (3584, 3968, 2), (5120, 4224, 2), (2048, 1024, 0),
+                                           (1040, 512, 0), (3584, 9472, 0)])
 def test_silu_mul_linear_equals_producer_then_gemm(gpu_lib, N, K, one_up_to):
     w, ws = synthetic.weights(N, K, seed=N + K)
     wq, sq = repacked(w, ws)
