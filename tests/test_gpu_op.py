@@ -312,3 +312,30 @@ def test_padded_cloned_output_and_debug_switches(kernel, monkeypatch, capsys):
     err = capsys.readouterr().err
     lines = [ln for ln in err.splitlines() if ln.startswith("[radiance.mxfp4.exact]")]
     assert len(lines) == 4 and all(ln.endswith(" ok") for ln in lines), err
+
+
+@pytest.mark.parametrize("M", [0, 3])
+def test_bodies_return_new_tensors(kernel, M):
+    """What custom_op checks on the public op and the direct registration does not: no output of a
+    body is an input or shares its memory, on an empty batch either."""
+    F, N, K = radiance_fused_norm, 64, 512
+    layer = Layer(*synthetic.weights(N, K, seed=5))
+    kernel.process_weights_after_loading(layer)
+    x, wide = bf16_dev(synthetic.activations(3, K, seed=6))[:M], \
+        bf16_dev(synthetic.activations(3, 2 * K, seed=7))[:M]
+    bias = torch.randn(N, device="cuda").bfloat16()
+    head = bias.repeat(2)
+    q, s = R.quant_per_token(x)
+    weights = (layer.weight, layer.weight_scale, layer.radiance_wref)
+    for body, args in [(R._mxfp4_linear, (x, *weights)), (R._mxfp4_linear_bias, (x, *weights, bias)),
+                       (R._mxfp4_linear_bias, (x, *weights, head[1:N + 1])),
+                       (R._mxfp4_linear_pq, (q, s, *weights)),
+                       (R._silu_mul_mxfp4_linear, (wide, *weights)),
+                       (F._add_rms_quant, (x, x, wide.new_ones(K), 1e-6)), (F._silu_mul_quant, (wide,)),
+                       (F._gdn_norm_quant, (x, x, head, 1e-6))]:
+        out = body(*args)
+        ins = [a for a in args if isinstance(a, torch.Tensor)]
+        for o in out if isinstance(out, tuple) else (out,):
+            assert all(o is not a for a in ins), body.__name__
+            assert not o.numel() or all(o.untyped_storage().data_ptr() != a.untyped_storage().data_ptr()
+                                        for a in ins), body.__name__
