@@ -648,7 +648,10 @@ def test_read_probe_reads_without_writing(gpu_lib, nbytes):
 
 
 @pytest.mark.parametrize("M,N,K", [(8, 17408, 5120), (1, 10240, 5120), (8, 5120, 8704),
-                                   (4, 5120, 6144), (3, 1000, 1024)])
+                                   (4, 5120, 6144), (3, 1000, 1024),
+                                   # a last k-group of 2, 3, 1 and 2 k-tiles; 4-, 10- and 16-wave plans
+                                   (8, 5120, 4352), (5, 2048, 3968), (1, 300, 4224), (8, 3584, 9472),
+                                   (8, 17408, 4352)])
 def test_stream_load_probe_runs_without_writing(gpu_lib, M, N, K):
     """The streaming GEMM's loads alone, each load set, on operands of the GEMM's own sizes (zero
     data never xors to the pattern): it runs and writes nothing; a shape the plan does not stream
@@ -707,7 +710,10 @@ NAN_SCALES = [0x7FC00000, 0xFFC00000, 0x7FC12345, 0xFFFFFFFF, 0x7F800001]
     (8, 512, 1024, 0, -1, 0, "stream"),
     (40, 17408, 5120, 0, -1, 0, "band"),
     (256, 1024, 1024, TILE, 2, 1, "tile, full tiles (staged stores)"),
-    (200, 1000, 1024, TILE, 2, 1, "tile, edge tiles (direct stores)"),
+    (200, 1000, 1024, TILE, 2, 1, "tile, edge tiles (staged stores)"),
+    (200, 1004, 1024, TILE, 2, 1, "tile, 8-byte direct stores"),
+    (200, 1003, 1024, TILE, 2, 1, "tile, scalar direct stores"),
+    (16, 1000, 640, 0, -1, 0, "skinny"),
     (24, 5120, 8704, 0, -1, 0, "tile K split + reduce"),
 ])
 def test_nan_token_scales_give_canonical_nan_rows(gpu_lib, M, N, K, kernel, variant, split, path):
@@ -724,8 +730,9 @@ def test_nan_token_scales_give_canonical_nan_rows(gpu_lib, M, N, K, kernel, vari
     print(f"[kernels] NaN token scales, {path}, M={M} N={N} K={K}", flush=True)
     c = gpu_gemm(q, s, wq, sq, N, K, kernel, variant, split)
     if kernel == 0:
-        assert _native.plan(M, N, K)[0] == {"stream": STREAM, "band": _native.KERNEL_BAND}.get(
-            path, TILE), _native.plan(M, N, K)
+        assert _native.plan(M, N, K)[0] == {"stream": STREAM, "band": _native.KERNEL_BAND,
+                                            "skinny": _native.KERNEL_SKINNY}.get(path, TILE), \
+            _native.plan(M, N, K)
     for r, bits in zip(rows, NAN_SCALES):
         want = 0x7FC0 | ((bits >> 16) & 0x8000)
         assert (c[r] == want).all(), (path, r, hex(bits), np.unique(c[r])[:4])
