@@ -93,9 +93,13 @@ __device__ __forceinline__ uint32_t bf16x2_rne(float lo, float hi) {
 // Two rounded bf16 outputs plus two bf16 biases, rounded again: the bits of an elementwise bf16 add
 // after the GEMM, without its launch and its pass over the output. Measured on MI355X, one token
 // count of a decode batch: N = 5120 K = 4352 M = 13, quantizer + GEMM + bias, 11.2 -> 8.35 us.
+// That add gives 0x7FC0 for every NaN, without a sign: the rounded sum's NaN halves are 0x7FC0 under
+// their sign and no other half has so large a magnitude, so adding 0x0040 to the magnitudes carries
+// into bit 15 for NaNs alone, and clears their sign there.
 __device__ __forceinline__ uint32_t add_bias2(uint32_t y, uint32_t bias) {
-  return bf16x2_rne(__uint_as_float(y << 16) + __uint_as_float(bias << 16),
-                    __uint_as_float(y & 0xFFFF0000u) + __uint_as_float(bias & 0xFFFF0000u));
+  const uint32_t r = bf16x2_rne(__uint_as_float(y << 16) + __uint_as_float(bias << 16),
+                                __uint_as_float(y & 0xFFFF0000u) + __uint_as_float(bias & 0xFFFF0000u));
+  return r & ~(((r & 0x7FFF7FFFu) + 0x00400040u) & 0x80008000u);
 }
 // the same for columns n .. n + 3 (n % 4 == 0; bias 16-byte aligned, N values)
 __device__ __forceinline__ uint2 add_bias4(uint2 y, const uint16_t* bias, int n, int N) {
