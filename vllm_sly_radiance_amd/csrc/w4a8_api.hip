@@ -175,10 +175,11 @@ int find_stream(int M, int N, int K, int dev) {
 // one tile per CU that the shape takes (1, 2 or 3; more in proportion to 3).
 // ns per slab on MI355X, medians over 8 decoder shapes (N 3584 .. 28672, K 3584 .. 9472) at M = 65,
 // 80, 96, 128, 160, 192, 200, 224, 256, 320, 384, 448, 512, 640, 768, 900 and 1024, weights
-// rotating through 400 MB, after 4 us of launch, first fill and epilogue. At these M a slab is
-// bound by LDS traffic (a 128 x 128 slab moves 64 KiB of fragment reads and 24 KiB of fills
-// through LDS against ~215 ns of MFMA), so tiles whose waves own more columns per token row (a
-// column is 64 bytes of a slab, a token 128) and that read their fragments a slab ahead do best.
+// rotating through 400 MB, after 4 us of launch, first fill and epilogue. At these M no unit of a
+// CU is busy (counters at M = 200 .. 1111: matrix cores 17-44 % of the cycles, LDS reads 11-21 %);
+// a slab is a chain of fill latency, barrier, fragment reads and MFMAs on one or two waves per
+// SIMD. Tiles that move fewer bytes per MFMA (a column is 64 bytes of a slab, a token 128) and
+// read their fragments a slab ahead do best.
 // Against the fastest tile at each of the 136 points the pick is 0.4 % slower on average; a table
 // of one throughput per tile, the rule before, picked 7 % slower ones (N = 17408 M = 200 31.7
 // against 27.5 us, N = 10240 M = 200 / 512 21.4 / 32.7 against 17.4 / 27.9, N = 5120 K = 8704

@@ -32,13 +32,15 @@
 //  * Epilogue: a lane holds 4 consecutive columns of one token; scaled by the per-token fp32 scale,
 //    rounded to bf16 and stored 8 bytes at a time.
 //  * AH = true reads every fragment one slab ahead, between the MFMAs of the slab before, so the
-//    LDS reads of a slab (64 KiB for 128 x 128 in 8 waves, ~250 ns) run under the MFMAs of the one
-//    before instead of in front of their own. Measured on MI355X (us, same bits): 128 x 128 in 8
-//    waves at N = 5120 K = 6144 M = 512 23.6 -> 22.0, N = 10240 M = 200 21.1 -> 19.9; 64 x 128 in 4
-//    waves at N = 5120 K = 6144 M = 200 16.7 -> 15.9; no gain up to 64 tokens, where the tiles are
-//    bound by their fills. The mid-M tiles use it (96 x 128, 64 x 96, 64 x 160 in 4 waves and
-//    128 x 128, 128 x 160, 128 x 192 in 8); the 256-row tiles keep the WM >= 3 pipeline, which needs
-//    fewer registers (256 x 256 ahead in 4 waves spilled 109 and took 734 us against 281).
+//    latency of a slab's LDS reads runs under the MFMAs of the one before instead of in front of
+//    their own. Their bandwidth is not the matter: a ds_read_b128 takes 4 clocks (525 bytes per
+//    ns and CU in a loop of reads), so the 64 KiB that 128 x 128 reads per slab in 8 waves take
+//    256. Measured on MI355X (us, same bits): 128 x 128 in 8 waves at N = 5120 K = 6144 M = 512
+//    23.6 -> 22.0, N = 10240 M = 200 21.1 -> 19.9; -1 .. +3 % on the tiles up to 64 tokens, which
+//    keep the plain order (64 x 128, the widest of them, is priced above 64 tokens as it is). The
+//    mid-M tiles use it (96 x 128, 64 x 96, 64 x 160 in 4 waves and 128 x 128, 128 x 160, 128 x 192
+//    in 8); the 256-row tiles keep the WM >= 3 pipeline, which needs fewer registers (256 x 256
+//    ahead in 4 waves spilled 109 and took 734 us against 281).
 //  * AT = true reads the activations in the fragment-tiled layout the producers can write (16-token
 //    blocks of 16 x K bytes; in block b, k-tile t, half h, lane l's 16 bytes at
 //    ((b KT + t) 2 + h) 1024 + 16 l are token 16 b + l % 16, k-bytes 128 t + 16 (4 h + l / 16)):
@@ -624,7 +626,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_tile_split(
 
 
 // (WM, WN, NS, NW, AH): NW waves of 16 WM x 16 WN in an (NW / 2) x 2 arrangement, NS-stage LDS
-// pipeline, AH 1 with every fragment read a slab ahead (LDS = NS * STAGE + ring_slots(NS) scale slots + token scales <= 160 KiB)
+// pipeline, AH 1 with every fragment read a slab ahead (LDS = NS * STAGE + ring_slots(NS) scale
+// slots + token scales <= 160 KiB). A variant's index is its name in forced plans, so variants that
+// no automatic plan takes any more stay where they are.
 #define W4A8_TILE_TABLE(X)                                                                        \
   X(2, 4, 4, 4, 0) X(4, 4, 3, 4, 0) X(4, 4, 4, 4, 0) X(8, 4, 3, 4, 0) X(4, 8, 3, 4, 0)            \
   X(8, 8, 3, 4, 0) X(8, 5, 3, 4, 0) X(4, 8, 4, 4, 0) X(4, 2, 4, 4, 0) X(1, 2, 4, 4, 0)            \
