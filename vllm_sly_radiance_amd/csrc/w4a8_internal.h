@@ -81,25 +81,26 @@ __device__ __forceinline__ v8i load_x_frag(const uint8_t* row, int k0, int g, in
 typedef __bf16 w4a8_bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float w4a8_f32x2_t __attribute__((ext_vector_type(2)));
 typedef unsigned short w4a8_u16x2_t __attribute__((ext_vector_type(2)));
+// SIGNLESS: every NaN as 0x7FC0, the bits of torch's rounding. Adding 0x0040 to the magnitudes
+// carries into bit 15 of the canonical NaNs alone, which masks their sign out.
+template <bool SIGNLESS = false>
 __device__ __forceinline__ uint32_t bf16x2_rne(float lo, float hi) {
   const uint32_t r =
       __builtin_bit_cast(uint32_t, __builtin_convertvector(w4a8_f32x2_t{lo, hi}, w4a8_bf16x2_t));
   const w4a8_u16x2_t mag = __builtin_bit_cast(w4a8_u16x2_t, r & 0x7FFF7FFFu);
   const uint32_t m = __builtin_bit_cast(
       uint32_t, __builtin_elementwise_min(mag, w4a8_u16x2_t{0x7FC0, 0x7FC0}));
+  if constexpr (SIGNLESS) return (r & ~(m + 0x00400040u) & 0x80008000u) | m;
   return (r & 0x80008000u) | m;
 }
 
 // Two rounded bf16 outputs plus two bf16 biases, rounded again: the bits of an elementwise bf16 add
 // after the GEMM, without its launch and its pass over the output. Measured on MI355X, one token
 // count of a decode batch: N = 5120 K = 4352 M = 13, quantizer + GEMM + bias, 11.2 -> 8.35 us.
-// That add gives 0x7FC0 for every NaN, without a sign: the rounded sum's NaN halves are 0x7FC0 under
-// their sign and no other half has so large a magnitude, so adding 0x0040 to the magnitudes carries
-// into bit 15 for NaNs alone, and clears their sign there.
+// That add gives 0x7FC0 for every NaN (SIGNLESS).
 __device__ __forceinline__ uint32_t add_bias2(uint32_t y, uint32_t bias) {
-  const uint32_t r = bf16x2_rne(__uint_as_float(y << 16) + __uint_as_float(bias << 16),
-                                __uint_as_float(y & 0xFFFF0000u) + __uint_as_float(bias & 0xFFFF0000u));
-  return r & ~(((r & 0x7FFF7FFFu) + 0x00400040u) & 0x80008000u);
+  return bf16x2_rne<true>(__uint_as_float(y << 16) + __uint_as_float(bias << 16),
+                          __uint_as_float(y & 0xFFFF0000u) + __uint_as_float(bias & 0xFFFF0000u));
 }
 // the same for columns n .. n + 3 (n % 4 == 0; bias 16-byte aligned, N values)
 __device__ __forceinline__ uint2 add_bias4(uint2 y, const uint16_t* bias, int n, int N) {
